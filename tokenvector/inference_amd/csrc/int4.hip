@@ -8,7 +8,8 @@
 //                      the pair coded with the scale of group c / group_size
 //                      as in the reference).  Unpack: one lane per byte.
 //   INT4 GEMM          y = fl32(sum_k x * ((nibble - 8) * scale) + bias) with
-//                      f64 accumulation on v_mfma_f64_16x16x4_f64: 64 x 64
+//                      f64 accumulation.  Large products: int4_planes.hip.
+//                      Here, on v_mfma_f64_16x16x4_f64: 64 x 64
 //                      tiles (operands straight into MFMA fragments, or
 //                      staged in LDS for the act-order gather), K split over
 //                      workgroups when the tiles are few; decode batches of
@@ -184,6 +185,32 @@ __global__ __launch_bounds__(kI4Block) void k_permute_cols(const float* __restri
         } else {
             out[i] = ok ? src[r * cols + p] : 0.0f;
         }
+    }
+}
+
+// The gather form for cols <= kPermCols: a block takes ROWS whole rows through
+// LDS, so that every line of src is read once and in order (read straight from
+// memory, each element fetches a line of its own), and reads perm once for
+// them.  8192 x 3072: 133 -> 60 us.
+constexpr int kPermCols = 16384;
+
+template <int ROWS>
+__global__ __launch_bounds__(kI4Block) void k_permute_rows(const float* __restrict__ src,
+                                                           int64_t rows, int cols,
+                                                           const int64_t* __restrict__ perm,
+                                                           float* __restrict__ out) {
+    extern __shared__ float s_row[];
+    for (int64_t r0 = (int64_t)blockIdx.x * ROWS; r0 < rows; r0 += (int64_t)gridDim.x * ROWS) {
+        const int n = (int)(rows - r0 < ROWS ? rows - r0 : ROWS);
+        for (int i = threadIdx.x; i < n * cols; i += kI4Block) s_row[i] = src[r0 * cols + i];
+        __syncthreads();
+        for (int c = threadIdx.x; c < cols; c += kI4Block) {
+            const int64_t p = perm[c];
+            const bool ok = p >= 0 && p < cols;
+            for (int r = 0; r < n; r++)
+                out[(r0 + r) * cols + c] = ok ? s_row[r * cols + (int)p] : 0.0f;
+        }
+        __syncthreads();
     }
 }
 
@@ -946,6 +973,20 @@ int launch_int4_dequantize(Ctx* c, const void* packed, bool in32, int64_t rows, 
 int launch_permute_cols(Ctx* c, const float* src, int64_t rows, int64_t cols, const int64_t* perm,
                         bool inverse, float* out) {
     if (rows * cols <= 0) return TKV_HIP_OK;
+    if (!inverse && cols <= kPermCols) {
+        const bool four = cols <= kPermCols / 4;
+        int64_t blocks = ceil_div(rows, (int64_t)(four ? 4 : 1));
+        if (blocks > (int64_t)c->num_cus * 8) blocks = (int64_t)c->num_cus * 8;
+        const unsigned lds = (unsigned)(cols * 4 * (four ? 4 : 1));
+        if (four)
+            hipLaunchKernelGGL(k_permute_rows<4>, dim3((unsigned)blocks), dim3(kI4Block), lds,
+                               c->stream, src, rows, (int)cols, perm, out);
+        else
+            hipLaunchKernelGGL(k_permute_rows<1>, dim3((unsigned)blocks), dim3(kI4Block), lds,
+                               c->stream, src, rows, (int)cols, perm, out);
+        TKV_LAUNCH_CHECK();
+        return TKV_HIP_OK;
+    }
     const unsigned g = grid_for(c, rows * cols);
     if (inverse)
         hipLaunchKernelGGL(k_permute_cols<true>, dim3(g), dim3(kI4Block), 0, c->stream, src, rows,
@@ -953,6 +994,16 @@ int launch_permute_cols(Ctx* c, const float* src, int64_t rows, int64_t cols, co
     else
         hipLaunchKernelGGL(k_permute_cols<false>, dim3(g), dim3(kI4Block), 0, c->stream, src, rows,
                            cols, perm, out);
+    TKV_LAUNCH_CHECK();
+    return TKV_HIP_OK;
+}
+
+int launch_int4_split_sum(Ctx* c, const double* part, int splits, int64_t mt, int64_t nt,
+                          const float* bias, float* y, int m, int n) {
+    int64_t rblocks = ceil_div((int64_t)m * n, (int64_t)256);
+    if (rblocks > (int64_t)c->num_cus * 8) rblocks = (int64_t)c->num_cus * 8;
+    hipLaunchKernelGGL(k_int4_split_sum, dim3((unsigned)rblocks), dim3(256), 0, c->stream, part,
+                       splits, mt, nt, bias, y, m, n);
     TKV_LAUNCH_CHECK();
     return TKV_HIP_OK;
 }
@@ -1057,6 +1108,22 @@ int launch_matmul_int4(Ctx* c, const float* a, const uint8_t* wp, const float* s
         TKV_GEMV(32)
 #undef TKV_GEMV
     }
+    // Prefill on the INT8 MFMA through digit planes.  The prepass and the
+    // second launch cost ~8 us (~15 with a permutation), so it pays from about
+    // 1.6e8 multiply-adds; with smaller groups, which fold more often, from
+    // 2.6e8 (64) or 3.5e8 (32), unless a permutation sends the f64 form
+    // through its slower gather.  f64 MFMA -> planes: 768 x 768 M = 256 17.6
+    // -> 18.5 us, M = 384 22.1 -> 20.4; 768 x 3072 M = 64 21.1 -> 21.0; group
+    // size 64, 1126 x 768 M = 254 20.7 -> 23.2, M = 346 28.0 -> 23.4; 32, M =
+    // 346 28.2 -> 29.6, M = 462 32.6 -> 29.7, permuted M = 254 39.7 -> 32.8.
+    // 2304 x 768 M = 2048 140 -> 39 us, 3072 x 768 M = 8192 656 -> 131 us,
+    // 768 x 3072 M = 8192 permuted 4174 -> 244 us.
+    const double macs = (double)m * (double)n * (double)k;
+    if (macs >= (perm || gs >= 128 ? 1.6e8 : gs >= 64 ? 2.6e8 : 3.5e8)) {
+        const int rc = launch_matmul_int4_planes(c, a, wp, scales, bias, perm, y, m, n, k, gs);
+        // no memory for the planes: the kernels below need far less
+        if (rc != TKV_HIP_UNSUPPORTED && rc != TKV_HIP_OOM) return rc;
+    }
     const dim3 grid((unsigned)((n + kGBN - 1) / kGBN), (unsigned)((m + kGBM - 1) / kGBM));
     const bool vec = !perm && k > 0 && k % 8 == 0 && gs % 8 == 0 && aligned(a, 16) && aligned(wp, 4);
     // K split over workgroups (f64 partial tiles that k_int4_split_sum adds
@@ -1121,12 +1188,7 @@ int launch_matmul_int4(Ctx* c, const float* a, const uint8_t* wp, const float* s
                                wp, scales, bias, perm, y, (int)m, (int)n, (int)k, (int)gs,
                                (int)kchunk, dp);
         TKV_LAUNCH_CHECK();
-        int64_t rblocks = ceil_div(m * n, (int64_t)256);
-        if (rblocks > (int64_t)c->num_cus * 8) rblocks = (int64_t)c->num_cus * 8;
-        hipLaunchKernelGGL(k_int4_split_sum, dim3((unsigned)rblocks), dim3(256), 0, c->stream, dp,
-                           (int)splits, mt, nt, bias, y, (int)m, (int)n);
-        TKV_LAUNCH_CHECK();
-        return TKV_HIP_OK;
+        return launch_int4_split_sum(c, dp, (int)splits, mt, nt, bias, y, (int)m, (int)n);
     }
     if (perm)
         hipLaunchKernelGGL((k_matmul_int4_f64<true>), grid, dim3(256), 0, c->stream, a, wp,

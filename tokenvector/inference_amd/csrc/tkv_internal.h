@@ -83,7 +83,9 @@ struct Ctx {
     unsigned long long* cal_hist = nullptr;
     unsigned* cal_arrivals = nullptr;
     // grow-only workspaces
-    static constexpr int kSlots = 13;  // 10, 11: f16-decoded FP8 operands; 12: INT4 split-K partials (either kernel)
+    // 10, 11: f16-decoded FP8 operands; 12: INT4 split-K partials (any kernel);
+    // 13, 14, 15: INT4 digit planes, retiled weight codes, permuted activations
+    static constexpr int kSlots = 16;
     void* ws[kSlots] = {};
     size_t ws_bytes[kSlots] = {};
     bool capturing = false;  // between capture_begin and capture_end
@@ -236,6 +238,16 @@ int launch_permute_cols(Ctx* c, const float* src, int64_t rows, int64_t cols, co
 int launch_matmul_int4(Ctx* c, const float* a, const uint8_t* wp, const float* scales,
                        const float* bias, const int64_t* perm, float* y, int64_t m, int64_t n,
                        int64_t k, int64_t gs);
+// The same on the INT8 MFMA through the activations' digit planes
+// (int4_planes.hip).  K not a multiple of 128 or above 65536, group sizes
+// other than 32, 64 and the multiples of 128, unaligned operands, or a capture
+// whose workspaces are too small: UNSUPPORTED, nothing launched.
+int launch_matmul_int4_planes(Ctx* c, const float* a, const uint8_t* wp, const float* scales,
+                              const float* bias, const int64_t* perm, float* y, int64_t m,
+                              int64_t n, int64_t k, int64_t gs);
+// y = fl32(part[0] + .. + part[splits - 1] + bias), f64 partials [mt, nt].
+int launch_int4_split_sum(Ctx* c, const double* part, int splits, int64_t mt, int64_t nt,
+                          const float* bias, float* y, int m, int n);
 // GGUF block decoding, dtype 8 (Q8_0), 2 (Q4_0) or 3 (Q4_1); bytes per
 // 32-element block (0 for any other dtype).
 int launch_gguf_blocks(Ctx* c, const uint8_t* raw, int64_t n, int dtype, float* out);
