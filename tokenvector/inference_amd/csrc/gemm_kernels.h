@@ -1013,6 +1013,13 @@ typedef CfgWS<128, 192, 4, 3, 128, 3, 4, 1, 1> Cfg9;  // Cfg8 + stores spread ov
 // stores overlap the other's K loop
 typedef Cfg<128, 192, 2, 2, 128, 2> Cfg11;  //  80 KB, 4 waves (64x96), two workgroups per CU
 
+// Few tiles for the CUs: a workgroup alone on its CU pays a slice's barrier,
+// DMA issue, LDS reads and MFMAs one after the other, so 256-byte slices (row
+// strides that are a multiple of it) halve the number of those chains.
+typedef Cfg<64, 64, 2, 2, 256, 4> Cfg12;    // 128 KB, 4 waves (32x32)
+typedef Cfg<128, 128, 4, 2, 256, 2> Cfg13;  // 128 KB, 8 waves (32x64)
+typedef Cfg<64, 128, 2, 4, 128, 3> Cfg14;   //  72 KB, 8 waves (32x32)
+
 constexpr int kBK = 128;
 
 template <class C>
@@ -1020,21 +1027,36 @@ static int64_t tiles_of(int64_t m, int64_t n) {
     return ceil_div(m, C::BM) * ceil_div(n, C::BN);
 }
 
-// Tile choice: the largest tile that still gives every CU work; the
-// context's TKV_HIP_TUNE_GEMM_CFG override (0..11; 2.. are the warp-
-// specialised configurations, 10 the skinny kernel for INT8 with M <= 32, 11
-// the fused-role kernel) forces one.
-static inline int pick_cfg(Ctx* c, int64_t m, int64_t n) {
+// Tile choice; the context's TKV_HIP_TUNE_GEMM_CFG override (0..11; 2.. are the
+// warp-specialised configurations, 10 the skinny kernel for INT8 with M <= 32,
+// 11 the fused-role kernel) forces one of those.
+static inline int pick_cfg(Ctx* c, int64_t m, int64_t n, int64_t ldk, bool f8) {
     const int64_t f = tuned(c, TKV_HIP_TUNE_GEMM_CFG);
     if (f >= 0) return (int)f;
-    // Warp-specialised 128x192 tiles (cfg 2) measured best over the four
-    // GPT-2 shapes at M = 8192 (warmed-up, interleaved medians); 64x128 tiles
-    // keep every CU busy when M is small.  The switch is at three quarters of
-    // the CUs: at M = 2048, qkv's 192 tiles ran 10.2 us with cfg 2 against
-    // 11.4 (FP8) / 12.5 (INT8) with cfg 0, while attn_out and mlp_down (64
-    // tiles) ran 6.2 / 13.8 us with cfg 0 against 8.9 / 19.1 (one box, two
-    // rounds, HIP events).
-    return tiles_of<Cfg2>(m, n) * 4 >= (int64_t)c->num_cus * 3 ? 2 : 0;
+    // From the smallest tiles up, as long as they leave no CU a second one
+    // (whole linears, us, cfg 0 / 2 before -> after; int8 per token unless
+    // said):
+    //   64x64    768x3072 M = 40 16.6 -> 13.2, M = 1024 19.8 -> 16.0 (FP8
+    //            reference products 40.4 -> 33.1, qlinear 18.3 -> 12.2),
+    //            2304x768 M = 300 9.8 -> 8.6
+    //   64x128   768x3072 M = 2048 22.7 -> 21.2 (FP8 ref. 44.4 -> 40.9, qlinear
+    //            18.6 -> 15.4)
+    // then 128x128 or the warp-specialised 128x192 by rounds over the CUs, a
+    // round of the smaller tile taking 0.77 of the larger's (measured 0.68 ..
+    // 0.79): 768x3072 M = 3001 (144 tiles against 96) qlinear 24.1 -> 21.3,
+    // 2304x768 M = 3001 (432 in two rounds against 288 in two) 22.8 -> 19.4;
+    // 128x192 stays for 2304x768 M = 2048 (14.9 against 18.9), 3072x768 M =
+    // 3001 (23.9 against 26.6) and large M.
+    const int64_t ncu = c->num_cus;
+    const bool wide_k = ldk % 256 == 0;
+    if (wide_k && tiles_of<Cfg12>(m, n) <= ncu) return 12;
+    if (tiles_of<Cfg14>(m, n) <= ncu) return 14;
+    const int64_t t2 = tiles_of<Cfg2>(m, n);
+    // (the FP8 policy holds a whole slice's fragments: 4-12% slower on it)
+    if (wide_k && !f8 && 77 * ceil_div(tiles_of<Cfg13>(m, n), ncu) < 100 * ceil_div(t2, ncu)) return 13;
+    // 128x192 tiles on three quarters of the CUs and up: at M = 2048, qkv's
+    // 192 ran 10.2 us with cfg 2 against 11.4 (FP8) / 12.5 (INT8) with cfg 0
+    return t2 * 4 >= ncu * 3 ? 2 : 0;
 }
 
 template <class C, class P, class E>
@@ -1182,7 +1204,7 @@ static int launch_gemv(Ctx* c, const uint8_t* a, const uint8_t* w, int64_t m, in
 template <class P, class E>
 static int launch_any(Ctx* c, const uint8_t* a, const uint8_t* w, int64_t m, int64_t n,
                       int64_t ldk, const E& ep, void* y) {
-    const int cfg = pick_cfg(c, m, n);
+    const int cfg = pick_cfg(c, m, n, ldk, std::is_same_v<P, PolicyF8>);
     const bool forced = tuned(c, TKV_HIP_TUNE_GEMM_CFG) >= 0;
     // The split sums need the warp-specialised kernel and 2 (BM WN + BN WM)
     // ints of LDS beside its ring (all of cfg 6's LDS is ring); other
@@ -1215,6 +1237,9 @@ static int launch_any(Ctx* c, const uint8_t* a, const uint8_t* w, int64_t m, int
         case 8: return launch_ws<Cfg8, P>(c, a, w, m, n, ldk, ep, y);
         case 9: return launch_ws<Cfg9, P>(c, a, w, m, n, ldk, ep, y);
         case 11: return launch_fused<Cfg11, P>(c, a, w, m, n, ldk, ep, y);
+        case 12: return launch_cfg<Cfg12, P>(c, a, w, m, n, ldk, ep, y);
+        case 13: return launch_cfg<Cfg13, P>(c, a, w, m, n, ldk, ep, y);
+        case 14: return launch_cfg<Cfg14, P>(c, a, w, m, n, ldk, ep, y);
         default: return launch_cfg<Cfg0, P>(c, a, w, m, n, ldk, ep, y);
     }
 }
