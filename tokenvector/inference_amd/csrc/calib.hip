@@ -620,6 +620,226 @@ constexpr MsePartialsFn mse_partials_for(int ch, std::integer_sequence<int, CH..
     return fns[ch - 1];
 }
 
+// ---- many elements, 16 .. 64 candidates: one pass over x ----
+// In units of u = am / (254 nc) candidate c's step is 2c, so its rounding
+// boundaries (q + 1/2) scale are the integers c (2q + 1): every boundary of
+// every candidate.  Between neighbouring ones (a bin) each candidate rounds all
+// elements to one code, and with y = |x| / u, start s_b and d = y - s_b
+//   sum (y - 2 c q)^2 = sum d^2 + t (n_b t + 2 sum d),   t = s_b - 2 c q,
+// q = min((s_b + c) / (2 c), 127) (integers), where sum d^2 needs no bins: it is
+// the same for every candidate.  So one pass counts n_b and adds d per bin
+// (LDS), and nc x bins terms replace nc x n.  d is added in fixed point (2^-F,
+// F chosen so that a block's sum stays below 2^63: 2^-41 at 6.3 M elements,
+// 2^-38 at 50 M), which makes the result independent of the order; elements
+// within rounding of a boundary are equally far from both codes.
+//   f64 VALU work falls from 350 operations per element to 8 (nc = 50), which
+// leaves the two LDS atomics: 6.3 M elements, whole call, 105 -> 36 us; 50 M,
+// 579 -> 97 us.
+constexpr int kMseHistMin = 16, kMseHistMax = 64;
+constexpr int kMseHistBlock = 1024;
+// At least the bins of nc candidates (the different integers c (2q + 1), and
+// one), counted for 16 .. 64: 1541 for 16, 2864 for 32, 4218 for 50, 5309 for 64.
+constexpr int mse_bin_cap(int nc) { return 80 * nc + 320; }
+constexpr int mse_cells(int nc) { return 254 * nc; }
+
+// Dynamic LDS: s1 u64 [cap], counts u32 [cap], lut u32 [cells].  Block b writes
+// its bins to rows b and its sum of d^2 to s2[b].  Every block reduces the min /
+// max partials and builds lut (cell j = int(y) -> bin | (j - start) << 16) for
+// itself from the marked boundaries, ~2 us; as a launch of its own, 13 us.  Block
+// 0 records starts[bin], *nbins and st.
+__global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
+    const float* __restrict__ x, int64_t n, int vec, int nc, int cap, double fixed, int nparts,
+    const RedPartial* __restrict__ partials, CalibState* __restrict__ st,
+    unsigned long long* __restrict__ rows_s1, uint32_t* __restrict__ rows_n,
+    double* __restrict__ s2, uint32_t* __restrict__ starts, int* __restrict__ nbins) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t s_mse[];
+    unsigned long long* s_s1 = reinterpret_cast<unsigned long long*>(s_mse);
+    uint32_t* s_n = reinterpret_cast<uint32_t*>(s_s1 + cap);
+    uint32_t* s_lut = s_n + cap;
+    constexpr int kWords = 512, kWaves = kMseHistBlock / 64;
+    static_assert(mse_cells(kMseHistMax) < 32 * kWords && kWords <= kMseHistBlock, "marks");
+    __shared__ uint32_t s_mark[kWords];
+    __shared__ int s_bin[kWords], s_last[kWords], s_wbin[kWaves], s_wlast[kWaves];
+    __shared__ double s_red[kWaves];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, cells = mse_cells(nc);
+    if (t < kWords) s_mark[t] = 0;
+    for (int i = t; i < cap; i += kMseHistBlock) {
+        s_s1[i] = 0;
+        s_n[i] = 0;
+    }
+    double dmn, dmx;
+    reduce_partials<false, kMseHistBlock>(x, nparts, 0, partials, dmn, dmx);  // and a barrier
+    const double am = dmn <= dmx ? fmax(fabs(dmn), fabs(dmx)) : 0.0;
+    for (int i = t; i < nc * 127; i += kMseHistBlock) {
+        const int e = (i / 127 + 1) * (2 * (i % 127) + 1);
+        atomicOr(&s_mark[e >> 5], 1u << (e & 31));
+    }
+    __syncthreads();
+    // per word: the boundaries up to its end, and the last of them
+    const uint32_t mark = t < kWords ? s_mark[t] : 0u;
+    int cnt = __popc(mark), last = mark ? 32 * t + 31 - __clz((int)mark) : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int a = __shfl_up(cnt, o, 64), b = __shfl_up(last, o, 64);
+        if (lane >= o) {
+            cnt += a;
+            last = last > b ? last : b;
+        }
+    }
+    if (lane == 63) {
+        s_wbin[wave] = cnt;
+        s_wlast[wave] = last;
+    }
+    __syncthreads();
+    for (int w = 0; w < wave; w++) {
+        cnt += s_wbin[w];
+        last = last > s_wlast[w] ? last : s_wlast[w];
+    }
+    if (t < kWords) {
+        s_bin[t] = cnt;
+        s_last[t] = last;
+    }
+    __syncthreads();
+    for (int j = t; j < cells; j += kMseHistBlock) {
+        const int w = j >> 5;
+        const uint32_t m = s_mark[w], below = m & (0xffffffffu >> (31 - (j & 31)));
+        const int bin = s_bin[w] - __popc(m) + __popc(below);
+        const int start =
+            below ? 32 * w + 31 - __clz((int)below) : (w > 0 ? s_last[w - 1] : 0);
+        s_lut[j] = (uint32_t)bin | (uint32_t)(j - start) << 16;
+        if (blockIdx.x == 0 && j == start) starts[bin] = (uint32_t)j;
+    }
+    if (blockIdx.x == 0 && t == 0) {
+        nan_first(x, dmn, dmx);
+        st->am = am;
+        st->mn = dmn;
+        st->mx = dmx;
+        *nbins = s_bin[kWords - 1] + 1;
+    }
+    const double inv = (double)cells / am;
+    __syncthreads();
+    double acc = 0.0;
+    auto add = [&](float v) {
+        const double y = (double)fabsf(v) * inv;
+        int j;
+        asm("v_cvt_i32_f64 %0, %1" : "=v"(j) : "v"(y));  // saturates; NaN -> 0
+        j = j < cells ? j : cells - 1;
+        const uint32_t e = s_lut[j];
+        const double d = (y - (double)j) + (double)(e >> 16);
+        acc = __builtin_fma(d, d, acc);  // NaN stays
+        const double f = __builtin_fma(d, fixed, 0x1p52);
+        atomicAdd(&s_s1[e & 0xffffu],
+                  (unsigned long long)(__double_as_longlong(f) & 0xfffffffffffffll));
+        atomicAdd(&s_n[e & 0xffffu], 1u);
+    };
+    const int64_t stride = (int64_t)gridDim.x * kMseHistBlock;
+    const int64_t tid = (int64_t)blockIdx.x * kMseHistBlock + threadIdx.x;
+    const int64_t n4 = vec ? n / 4 : 0;
+    const float4* __restrict__ x4 = reinterpret_cast<const float4*>(x);
+    int64_t i = tid;
+    for (; i + stride < n4; i += 2 * stride) {
+        const float4 u = x4[i], w = x4[i + stride];
+        add(u.x);
+        add(u.y);
+        add(u.z);
+        add(u.w);
+        add(w.x);
+        add(w.y);
+        add(w.z);
+        add(w.w);
+    }
+    for (; i < n4; i += stride) {
+        const float4 u = x4[i];
+        add(u.x);
+        add(u.y);
+        add(u.z);
+        add(u.w);
+    }
+    for (int64_t k = 4 * n4 + tid; k < n; k += stride) add(x[k]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc = acc + __shfl_xor(acc, o, 64);
+    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < kMseHistBlock / 64; w++) t = t + s_red[w];
+        s2[blockIdx.x] = t;
+    }
+    for (int k = threadIdx.x; k < cap; k += kMseHistBlock) {
+        rows_s1[(int64_t)blockIdx.x * cap + k] = s_s1[k];
+        rows_n[(int64_t)blockIdx.x * cap + k] = s_n[k];
+    }
+}
+
+// bins[2 b] = n_b, bins[2 b + 1] = sum d of bin b: a block takes 32 bins, its 8
+// thread groups every eighth row.
+__global__ __launch_bounds__(kCalBlock) void k_mse_bin_sums(
+    int rows, int cap, double unfixed, const unsigned long long* __restrict__ rows_s1,
+    const uint32_t* __restrict__ rows_n, double* __restrict__ bins) {
+    __shared__ double s_a[kCalBlock], s_b[kCalBlock];
+    const int b = blockIdx.x * 32 + (threadIdx.x & 31);
+    double cn = 0.0, cs = 0.0;
+    if (b < cap)
+#pragma unroll 4
+        for (int r = threadIdx.x >> 5; r < rows; r += kCalBlock / 32) {
+            cn = cn + (double)rows_n[(int64_t)r * cap + b];
+            cs = cs + (double)rows_s1[(int64_t)r * cap + b];
+        }
+    s_a[threadIdx.x] = cn;
+    s_b[threadIdx.x] = cs;
+    __syncthreads();
+    if (threadIdx.x < 32 && b < cap) {
+        for (int g = 1; g < kCalBlock / 32; g++) {
+            cn = cn + s_a[32 * g + threadIdx.x];
+            cs = cs + s_b[32 * g + threadIdx.x];
+        }
+        bins[2 * b] = cn;
+        bins[2 * b + 1] = cs * unfixed;
+    }
+}
+
+// mse[c - 1] of candidate c = blockIdx.x + 1 from the bins; the block that
+// arrives last picks, as in k_mse_reduce.
+__global__ __launch_bounds__(kCalBlock) void k_mse_bin_eval(
+    int64_t n, int nc, int rows, const double* __restrict__ s2, const double* __restrict__ bins,
+    const uint32_t* __restrict__ starts, const int* __restrict__ nbins, double* __restrict__ mse,
+    const CalibState* __restrict__ st, unsigned* __restrict__ arrivals,
+    tkv_hip_qparams_dev* __restrict__ out) {
+    __shared__ double s_red[kCalBlock / 64];
+    const int c = (int)blockIdx.x + 1, nb = *nbins;
+    double a = 0.0;
+    for (int r = threadIdx.x; r < rows; r += kCalBlock) a = a + s2[r];
+    // (s + c) / (2 c) is at least 1/512 below the next integer once 1/2 is added
+    // to s + c; 2^-16 covers the product's rounding
+    const float half = 0.5f / (float)c;
+#pragma unroll 6
+    for (int b = threadIdx.x; b < nb; b += kCalBlock) {
+        const int s = (int)starts[b], q = min((int)(((float)(s + c) + 0.5f) * half), 127);
+        const double t = (double)(s - 2 * c * q);
+        a = __builtin_fma(t, __builtin_fma(bins[2 * b], t, 2.0 * bins[2 * b + 1]), a);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) a = a + __shfl_xor(a, o, 64);
+    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = a;
+    __syncthreads();
+    const double am = st->am, u = am / (double)mse_cells(nc);
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < kCalBlock / 64; w++) t = t + s_red[w];
+        __hip_atomic_store(mse + c - 1, t * u * u / (double)n, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!arrive_last(arrivals, gridDim.x)) return;
+    const int bc = block_first_min(mse, nc);
+    if (threadIdx.x == 0) {
+        if (am < 0.00000001)
+            finalize_minmax(st->mn, st->mx, MM_SYMMETRIC, TKV_HIP_RECIPE_PRIMARY, out);
+        else
+            write_sym(bc >= 0 ? am * (double)(bc + 1) / (double)nc : am, out);
+    }
+    arrive_clear(arrivals);
+}
+
 // mse[c] = (sum over the per-block partials, a fixed tree order) / n.  The
 // block that arrives last (arrive_last) makes the reference's first-minimum
 // pick over c ascending and writes the parameters.
@@ -664,7 +884,7 @@ int64_t hist_grid(Ctx* c, int64_t n) {
     return blocks < 1 ? 1 : blocks;
 }
 
-// Workspace slot 9: [CalibState][histogram or MSE table + partials].
+// Workspace slot 9: [CalibState][histogram, MSE table + partials, or MSE bins].
 int cal_workspace(Ctx* c, size_t extra, CalibState** st, void** rest) {
     void* w;
     TKV_RC_TRY(ctx_workspace(c, 9, 256 + extra, &w));
@@ -746,12 +966,67 @@ int launch_calibrate_percentile(Ctx* c, const float* x, int64_t n, float percent
     return TKV_HIP_OK;
 }
 
+// Below, the pass per 13 candidates is as fast: 50 candidates 2^17 elements
+// 32.9 -> 23.2 us, 32 candidates 23.3 -> 21.3; with fewer, 2^19 (16 candidates
+// 18.9 -> 22.1, 26 candidates 25.0 -> 24.7), 2^20 24.9 -> 23.9 and 33.0 -> 27.1.
+inline int64_t mse_hist_from(int nc) { return nc >= 32 ? 1 << 17 : 1 << 20; }
+// Fixed point has fewer bits for more elements; from here on f64 sums are the
+// more exact ones.
+constexpr int64_t kMseHistTo = (int64_t)1 << 30;
+
+static int calibrate_mse_hist(Ctx* c, const float* x, int64_t n, int nc,
+                              tkv_hip_qparams_dev* out) {
+    const int cells = mse_cells(nc), cap = mse_bin_cap(nc);
+    int64_t blocks = ceil_div(n, (int64_t)kMseHistBlock * 4);
+    if (blocks > c->num_cus) blocks = c->num_cus;
+    const int grid = (int)blocks;
+    // a block's elements, each below 2^7 (the widest bin is 2 nc cells): the
+    // fixed-point sum of all of them stays below 2^63
+    const int64_t most = (ceil_div(n, 4 * blocks * kMseHistBlock) + 1) * 4 * kMseHistBlock;
+    int bits = 0;
+    while (((int64_t)1 << bits) < most) bits++;
+    const double fixed = (double)(1ull << (56 - bits < 44 ? 56 - bits : 44));
+    const size_t need = (size_t)grid * cap * 12 + (size_t)grid * 8 + (size_t)cap * 20 +
+                        (size_t)nc * 8 + 64;
+    if (c->capturing && c->ws_bytes[9] < 256 + need) return TKV_HIP_UNSUPPORTED;
+    CalibState* st;
+    void* rest;
+    TKV_RC_TRY(cal_workspace(c, need, &st, &rest));
+    auto* rows_s1 = static_cast<unsigned long long*>(rest);
+    auto* bins = reinterpret_cast<double*>(rows_s1 + (size_t)grid * cap);
+    double* s2 = bins + 2 * cap;
+    double* mse = s2 + grid;
+    auto* rows_n = reinterpret_cast<uint32_t*>(mse + nc);
+    uint32_t* starts = rows_n + (size_t)grid * cap;
+    int* nbins = reinterpret_cast<int*>(starts + cap);
+    int64_t nparts;
+    TKV_RC_TRY(launch_partials(c, x, n, 0, &nparts));
+    hipLaunchKernelGGL(k_mse_hist, dim3((unsigned)grid), dim3(kMseHistBlock),
+                       (size_t)cap * 12 + (size_t)cells * 4, c->stream, x, n,
+                       aligned(x, 16) ? 1 : 0, nc, cap, fixed, (int)nparts, c->partials, st,
+                       rows_s1, rows_n, s2, starts, nbins);
+    TKV_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_mse_bin_sums, dim3((unsigned)ceil_div(cap, 32)), dim3(kCalBlock), 0,
+                       c->stream, grid, cap, 1.0 / fixed, rows_s1, rows_n, bins);
+    TKV_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_mse_bin_eval, dim3((unsigned)nc), dim3(kCalBlock), 0, c->stream, n, nc,
+                       grid, s2, bins, starts, nbins, mse, st, c->cal_arrivals + 3, out);
+    TKV_LAUNCH_CHECK();
+    return TKV_HIP_OK;
+}
+
 int launch_calibrate_mse(Ctx* c, const float* x, int64_t n, int64_t num_candidates,
                          tkv_hip_qparams_dev* out) {
     if (n <= 0 || num_candidates > kMaxMseCandidates)
         return set_error(TKV_HIP_BAD_ARG, "calibrate_mse: needs n > 0, num_candidates <= 4096");
     TKV_RC_TRY(need_cal_scratch(c, "calibrate_mse"));
     const int nc = (int)(num_candidates < 4 ? 4 : num_candidates);
+    // what the histogram's larger workspace cannot take (memory, a capture that
+    // began before it grew) goes on below
+    if (nc >= kMseHistMin && nc <= kMseHistMax && n >= mse_hist_from(nc) && n < kMseHistTo) {
+        const int rc = calibrate_mse_hist(c, x, n, nc, out);
+        if (!no_room(rc)) return rc;
+    }
     // passes of ch <= kMseChunk candidates, as even as whole passes allow
     const int passes = (int)ceil_div((int64_t)nc, (int64_t)kMseChunk);
     const int ch = (int)ceil_div((int64_t)nc, (int64_t)passes);

@@ -1122,7 +1122,7 @@ int launch_matmul_int4(Ctx* c, const float* a, const uint8_t* wp, const float* s
     if (macs >= (perm || gs >= 128 ? 1.6e8 : gs >= 64 ? 2.6e8 : 3.5e8)) {
         const int rc = launch_matmul_int4_planes(c, a, wp, scales, bias, perm, y, m, n, k, gs);
         // no memory for the planes: the kernels below need far less
-        if (rc != TKV_HIP_UNSUPPORTED && rc != TKV_HIP_OOM) return rc;
+        if (!no_room(rc)) return rc;
     }
     const dim3 grid((unsigned)((n + kGBN - 1) / kGBN), (unsigned)((m + kGBM - 1) / kGBM));
     const bool vec = !perm && k > 0 && k % 8 == 0 && gs % 8 == 0 && aligned(a, 16) && aligned(wp, 4);

@@ -34,6 +34,14 @@ int fail_hip(hipError_t e, const char* what, const char* file, int line);
 
 #define TKV_LAUNCH_CHECK() TKV_HIP_TRY(hipGetLastError())
 
+// A launcher that found no memory for its workspaces (or, inside a capture, no
+// room in them): its caller then takes the form that needs less.  hipMalloc's
+// error is taken off, or the next TKV_LAUNCH_CHECK would report it.
+inline bool no_room(int rc) {
+    if (rc == TKV_HIP_OOM) (void)hipGetLastError();
+    return rc == TKV_HIP_OOM || rc == TKV_HIP_UNSUPPORTED;
+}
+
 // ---------------------------------------------------------------------------
 // Context: device, stream, grow-only workspaces.  A context is driven by one
 // thread at a time; the default context of each thread is thread_local.

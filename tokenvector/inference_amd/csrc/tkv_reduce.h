@@ -147,26 +147,26 @@ __device__ __forceinline__ RedPartial load_partial(const RedPartial* p) {
     }
 }
 
-// Reduces the per-block partials (every thread of a kBlock-thread block
+// Reduces the per-block partials (every thread of a BLOCK-thread block
 // takes part; the result is returned to all of them) to the reference's f64
 // min / max locals.  The reference keeps the first element reaching an
 // extreme; values that compare equal are bit-identical except +-0, so a zero
 // extreme takes the sign of the first zero in index order.  SC1: partials
 // written by other workgroups of the running kernel (store_partial_sc1).
-template <bool SC1 = false>
+template <bool SC1 = false, int BLOCK = kBlock>
 __device__ inline void reduce_partials(const float* __restrict__ x, int nparts, int track_zero,
                                        const RedPartial* __restrict__ partials, double& dmn,
                                        double& dmx) {
     float mn = __builtin_inff(), mx = -__builtin_inff();
     unsigned long long zi = ~0ull;
-    for (int b = threadIdx.x; b < nparts; b += kBlock) {
+    for (int b = threadIdx.x; b < nparts; b += BLOCK) {
         const RedPartial p = load_partial<SC1>(partials + b);
         mn = fminf(mn, p.mn);
         mx = fmaxf(mx, p.mx);
         zi = p.zidx < zi ? p.zidx : zi;
     }
-    __shared__ float s_mn[kBlock / 64], s_mx[kBlock / 64];
-    __shared__ unsigned long long s_zi[kBlock / 64];
+    __shared__ float s_mn[BLOCK / 64], s_mx[BLOCK / 64];
+    __shared__ unsigned long long s_zi[BLOCK / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     mn = wave_min(mn);
     mx = wave_max(mx);
@@ -180,7 +180,7 @@ __device__ inline void reduce_partials(const float* __restrict__ x, int nparts, 
     mn = s_mn[0];
     mx = s_mx[0];
     zi = s_zi[0];
-    for (int w = 1; w < kBlock / 64; w++) {
+    for (int w = 1; w < BLOCK / 64; w++) {
         mn = fminf(mn, s_mn[w]);
         mx = fmaxf(mx, s_mx[w]);
         zi = s_zi[w] < zi ? s_zi[w] : zi;
