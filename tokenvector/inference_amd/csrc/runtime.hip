@@ -135,6 +135,12 @@ int ctx_destroy(Ctx* c) {
         if (c->ws[i]) (void)hipFree(c->ws[i]);
     for (void* p : c->retired) (void)hipFree(p);
     if (c->partials) (void)hipFree(c->partials);
+    for (hipEvent_t e : c->stage_event)
+        if (e) (void)hipEventDestroy(e);
+    if (c->stage_pinned)
+        (void)hipHostFree(c->stage);
+    else
+        free(c->stage);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
     return TKV_HIP_OK;
@@ -189,6 +195,38 @@ int ctx_workspace(Ctx* c, int slot, size_t bytes, void** out) {
         c->ws_bytes[slot] = sz;
     }
     *out = c->ws[slot];
+    return TKV_HIP_OK;
+}
+
+int ctx_stage_next(Ctx* c, void** half) {
+    if (c->capturing)
+        return set_error(TKV_HIP_BAD_ARG, "host arrays: not inside a stream capture");
+    for (hipEvent_t& e : c->stage_event)
+        if (!e) TKV_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (!c->stage) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, 2 * Ctx::kStageHalf, hipHostMallocDefault) == hipSuccess) {
+            c->stage_pinned = true;
+        } else {
+            (void)hipGetLastError();
+            p = malloc(2 * Ctx::kStageHalf);
+            if (!p) return set_error(TKV_HIP_OOM, "staging buffer: host allocation failed");
+        }
+        c->stage = static_cast<char*>(p);
+    }
+    if (c->stage_used[c->stage_at]) {
+        TKV_HIP_TRY(hipEventSynchronize(c->stage_event[c->stage_at]));
+        c->stage_used[c->stage_at] = false;
+    }
+    *half = c->stage + c->stage_at * Ctx::kStageHalf;
+    return TKV_HIP_OK;
+}
+
+int ctx_stage_sent(Ctx* c) {
+    // used from here on, also if the record fails: the next wait then reports it
+    c->stage_used[c->stage_at] = true;
+    TKV_HIP_TRY(hipEventRecord(c->stage_event[c->stage_at], c->stream));
+    c->stage_at ^= 1;
     return TKV_HIP_OK;
 }
 

@@ -96,6 +96,14 @@ struct Ctx {
     static constexpr int kSlots = 16;
     void* ws[kSlots] = {};
     size_t ws_bytes[kSlots] = {};
+    // Staging of the INT8 GEMM's host mirror: two halves of host memory, used
+    // in turn, each with the event of the last copy that reads or fills it.
+    static constexpr size_t kStageHalf = 256 << 10;
+    char* stage = nullptr;
+    bool stage_pinned = false;  // pageable where no pinned memory could be had
+    hipEvent_t stage_event[2] = {};
+    bool stage_used[2] = {};    // a copy since that half was last waited for
+    int stage_at = 0;           // the half that is used next
     bool capturing = false;  // between capture_begin and capture_end
     // Graphs captured on this context and not yet destroyed.  They replay
     // the workspace addresses they captured, so while any is alive a slot
@@ -123,6 +131,10 @@ int ctx_get(int64_t handle, Ctx** out);
 // Device workspace slot `slot` of at least `bytes` (contents undefined).
 // Refuses to grow while the context's stream is being captured.
 int ctx_workspace(Ctx* c, int slot, size_t bytes, void** out);
+// The next half of the staging buffer, after the last copy that used it;
+// ctx_stage_sent marks the copy just queued from or to it.
+int ctx_stage_next(Ctx* c, void** half);
+int ctx_stage_sent(Ctx* c);
 // Byte fill of [dst, dst + bytes) on the context's stream (a kernel).
 int launch_fill(Ctx* c, void* dst, int value, int64_t bytes);
 // Environment gate: TKV_QUANT_HIP=0 turns every host mirror into a
