@@ -396,6 +396,26 @@ int launch_quant_i8_tensor(Ctx* c, const float* x, int64_t n, const tkv_hip_qpar
     return TKV_HIP_OK;
 }
 
+// Four packed e4m3 bytes (element 0 in bits 7:0) as raw bytes (FP8_BYTES),
+// as the reference's int32 codes (byte - 128, FP8_I32), or as their exact
+// reference decode in f16, pre-scaled by 2^-8 (FP8_F16: what the
+// reference-products GEMM multiplies).
+enum { FP8_BYTES = 0, FP8_I32 = 1, FP8_F16 = 2 };
+
+template <int OUT>
+__device__ __forceinline__ void store_fp8x4(void* q, int64_t i4, uint32_t w) {
+    if constexpr (OUT == FP8_I32)
+        reinterpret_cast<int4*>(q)[i4] =
+            make_int4((int)(w & 0xffu) - 128, (int)((w >> 8) & 0xffu) - 128,
+                      (int)((w >> 16) & 0xffu) - 128, (int)(w >> 24) - 128);
+    else if constexpr (OUT == FP8_F16)
+        reinterpret_cast<uint2*>(q)[i4] =
+            make_uint2(gemm::dec2_f16(__builtin_amdgcn_perm(0u, w, 0x0c010c00u)),
+                       gemm::dec2_f16(__builtin_amdgcn_perm(0u, w, 0x0c030c02u)));
+    else
+        reinterpret_cast<uint32_t*>(q)[i4] = w;
+}
+
 // ---------------------------------------------------------------------------
 // Single-pass per-tensor calibrate + quantize for large tensors
 // (calibrate_minmax(x, 1), then quantize_int8_symmetric: engine.tkv:13-36,
@@ -406,7 +426,10 @@ int launch_quant_i8_tensor(Ctx* c, const float* x, int64_t n, const tkv_hip_qpar
 // crosses HBM once.  The two-kernel path reads it twice: at 8192 x 3072 it
 // takes 17.9 + 20.7 us, this kernel ~26 us (timestamped probe: loads 15-16
 // us at 6.3-6.8 TB/s, barrier ~3 us, codes ~7 us).  For a 25 MB tensor the
-// two were equal, so the kernel is used from kResMinElems up.
+// two were equal, so the kernel is used from kResMinElems up.  The FP8 forms
+// (MM_FP8 scale, e4m3 bytes or their f16 decode) hold x the same way: 32768 x
+// 768 in two kernels 13.2 + 20.7 us, the whole full-rate linear with N = 3072
+// 148.3 -> 138.9 us.
 //
 // Symmetric calibration needs only max(|min|, |max|), the absmax of the
 // elements that are not NaN (fmaxf skips NaN, as the reference's strict
@@ -455,8 +478,12 @@ __device__ __forceinline__ float block_max_res(float v, float* s) {
     return r;
 }
 
-template <bool OUT_I32>
-__global__ __launch_bounds__(kResBlock, 3) void k_quant_i8_resident(
+// What the single-pass kernel writes: int8 codes or their int32 form, e4m3
+// bytes, or the f16 decode of those (FP8_F16).
+enum { RES_I8 = 0, RES_I32 = 1, RES_FP8 = 2, RES_F16 = 3 };
+
+template <int OUT>
+__global__ __launch_bounds__(kResBlock, 3) void k_quant_resident(
     const float* __restrict__ x, int64_t n, tkv_hip_qparams_dev* __restrict__ p,
     void* __restrict__ q, int recipe, unsigned long long* __restrict__ slots, int spin) {
     __shared__ float4 s_x[kResLds * kResBlock];
@@ -551,24 +578,42 @@ __global__ __launch_bounds__(kResBlock, 3) void k_quant_i8_resident(
     double dmn = 0.0, dmx = (double)g;
     nan_first(x, dmn, dmx);
     tkv_hip_qparams_dev prm;
-    finalize_minmax(dmn, dmx, MM_SYMMETRIC, recipe, &prm);
-    const double inv = prm.inv;
+    constexpr bool kFp8 = OUT == RES_FP8 || OUT == RES_F16;
+    finalize_minmax(dmn, dmx, kFp8 ? MM_FP8 : MM_SYMMETRIC, recipe, &prm);
     if (blockIdx.x == 0 && threadIdx.x == 0) *p = prm;
-    auto store_codes = [&](auto&& code) {
+    auto each4 = [&](auto&& store) {
 #pragma unroll
         for (int u = 0; u < kResRegs; u++) {
             const int64_t i = tid + u * stride;
-            if (i < n4)
-                store4<OUT_I32>(q, i, code(v[u].x), code(v[u].y), code(v[u].z), code(v[u].w));
+            if (i < n4) store(i, v[u]);
         }
 #pragma unroll
         for (int u = 0; u < kResLds; u++) {
             const int64_t i = tid + (kResRegs + u) * stride;
-            if (i < n4) {
-                const float4 w = s_x[u * kResBlock + threadIdx.x];
-                store4<OUT_I32>(q, i, code(w.x), code(w.y), code(w.z), code(w.w));
-            }
+            if (i < n4) store(i, s_x[u * kResBlock + threadIdx.x]);
         }
+    };
+    if constexpr (kFp8) {
+        // as k_fp8_encode: x times the f32 reciprocal of the scale, then the
+        // e4m3 code, with the patched form where an element is inf or NaN
+        const float mul = 1.0f / prm.scale;
+        each4([&](int64_t i, float4 w) {
+            w.x *= mul;
+            w.y *= mul;
+            w.z *= mul;
+            w.w *= mul;
+            uint32_t code = e4m3_encode4_finite(w.x, w.y, w.z, w.w);
+            if (e4m3_special(w.x) || e4m3_special(w.y) || e4m3_special(w.z) || e4m3_special(w.w))
+                code = e4m3_encode4(w.x, w.y, w.z, w.w);
+            store_fp8x4<OUT == RES_F16 ? FP8_F16 : FP8_BYTES>(q, i, code);
+        });
+        return;
+    }
+    const double inv = prm.inv;
+    auto store_codes = [&](auto&& code) {
+        each4([&](int64_t i, const float4& w) {
+            store4<OUT == RES_I32>(q, i, code(w.x), code(w.y), code(w.z), code(w.w));
+        });
     };
     // The store phase is VALU-bound: with an f32 reciprocal (the primary
     // recipe's fl32(1 / scale)) the codes take the f32 form of the rounding
@@ -584,21 +629,24 @@ __global__ __launch_bounds__(kResBlock, 3) void k_quant_i8_resident(
 // TKV_HIP_UNSUPPORTED when the tensor is outside the single-pass kernel's
 // range (size, alignment, a tail of fewer than 4 elements) or the context
 // has no barrier slots.
-static int launch_quant_i8_resident(Ctx* c, const float* x, int64_t n, int recipe,
-                                    tkv_hip_qparams_dev* p, void* q, bool out_i32) {
+static int launch_quant_resident(Ctx* c, const float* x, int64_t n, int recipe,
+                                 tkv_hip_qparams_dev* p, void* q, int out) {
     const int64_t g = c->num_cus;
+    const int qalign = out == RES_I32 ? 16 : (out == RES_F16 ? 8 : 4);
     if (!c->grid_slots || g > kMaxGridSlots - 1 || n < kResMinElems || n % 4 != 0 ||
-        !aligned(x, 16) || !aligned(q, out_i32 ? 16 : 4) ||
+        !aligned(x, 16) || !aligned(q, qalign) ||
         n / 4 > g * kResBlock * (kResRegs + kResLds))
         return TKV_HIP_UNSUPPORTED;
     const int spin = tuned(c, TKV_HIP_TUNE_GRID_SPIN) >= 0 ? (int)tuned(c, TKV_HIP_TUNE_GRID_SPIN)
                                                            : kResSpin;
-    if (out_i32)
-        hipLaunchKernelGGL((k_quant_i8_resident<true>), dim3((unsigned)g), dim3(kResBlock), 0,
-                           c->stream, x, n, p, q, recipe, c->grid_slots, spin);
-    else
-        hipLaunchKernelGGL((k_quant_i8_resident<false>), dim3((unsigned)g), dim3(kResBlock), 0,
-                           c->stream, x, n, p, q, recipe, c->grid_slots, spin);
+#define TKV_RESIDENT(OUT)                                                                      \
+    hipLaunchKernelGGL((k_quant_resident<OUT>), dim3((unsigned)g), dim3(kResBlock), 0,        \
+                       c->stream, x, n, p, q, recipe, c->grid_slots, spin)
+    if (out == RES_I32) TKV_RESIDENT(RES_I32);
+    else if (out == RES_FP8) TKV_RESIDENT(RES_FP8);
+    else if (out == RES_F16) TKV_RESIDENT(RES_F16);
+    else TKV_RESIDENT(RES_I8);
+#undef TKV_RESIDENT
     TKV_LAUNCH_CHECK();
     return TKV_HIP_OK;
 }
@@ -611,7 +659,8 @@ int launch_quant_i8_dynamic(Ctx* c, const float* x, int64_t n, int recipe,
                             tkv_hip_qparams_dev* p, void* q, bool out_i32) {
     if (n <= 0) return launch_minmax_tensor(c, x, n, MM_SYMMETRIC, recipe, p);
     if (tuned(c, TKV_HIP_TUNE_QUANT_TWO_PASS) != 1) {
-        const int rc = launch_quant_i8_resident(c, x, n, recipe, p, q, out_i32);
+        const int rc = launch_quant_resident(c, x, n, recipe, p, q,
+                                             out_i32 ? RES_I32 : RES_I8);
         if (rc != TKV_HIP_UNSUPPORTED) return rc;
     }
     int64_t nparts;
@@ -903,26 +952,6 @@ int launch_dequant_i8(Ctx* c, const void* q, bool in_i32, int64_t rows, int64_t 
 // reference's int32 codes (byte - 128).  With `scaled` the input is first
 // multiplied by fl32(1 / scale) in f32 (extension for per-tensor FP8).
 // ---------------------------------------------------------------------------
-// Four packed e4m3 bytes (element 0 in bits 7:0) as raw bytes (FP8_BYTES),
-// as the reference's int32 codes (byte - 128, FP8_I32), or as their exact
-// reference decode in f16, pre-scaled by 2^-8 (FP8_F16: what the
-// reference-products GEMM multiplies).
-enum { FP8_BYTES = 0, FP8_I32 = 1, FP8_F16 = 2 };
-
-template <int OUT>
-__device__ __forceinline__ void store_fp8x4(void* q, int64_t i4, uint32_t w) {
-    if constexpr (OUT == FP8_I32)
-        reinterpret_cast<int4*>(q)[i4] =
-            make_int4((int)(w & 0xffu) - 128, (int)((w >> 8) & 0xffu) - 128,
-                      (int)((w >> 16) & 0xffu) - 128, (int)(w >> 24) - 128);
-    else if constexpr (OUT == FP8_F16)
-        reinterpret_cast<uint2*>(q)[i4] =
-            make_uint2(gemm::dec2_f16(__builtin_amdgcn_perm(0u, w, 0x0c010c00u)),
-                       gemm::dec2_f16(__builtin_amdgcn_perm(0u, w, 0x0c030c02u)));
-    else
-        reinterpret_cast<uint32_t*>(q)[i4] = w;
-}
-
 template <int OUT>
 __device__ __forceinline__ void store_fp8x1(void* q, int64_t j, uint32_t e) {
     if constexpr (OUT == FP8_I32)
@@ -1021,10 +1050,14 @@ int launch_fp8_encode(Ctx* c, const float* x, int64_t n, const tkv_hip_qparams_d
     return launch_fp8_encode_as(c, x, n, scaled, q, out_i32 ? FP8_I32 : FP8_BYTES);
 }
 
-// Per-tensor FP8 activation quantize: the MM_FP8 scale, then the scaled
-// encode reading it from *p.
+// Per-tensor FP8 activation quantize: the single-pass kernel where the tensor
+// fits it, else the MM_FP8 scale, then the scaled encode reading it from *p.
 int launch_quant_fp8_dynamic(Ctx* c, const float* x, int64_t n, tkv_hip_qparams_dev* p, void* q,
                              bool out_i32) {
+    if (!out_i32 && tuned(c, TKV_HIP_TUNE_QUANT_TWO_PASS) != 1) {
+        const int rc = launch_quant_resident(c, x, n, TKV_HIP_RECIPE_PRIMARY, p, q, RES_FP8);
+        if (rc != TKV_HIP_UNSUPPORTED) return rc;
+    }
     TKV_RC_TRY(launch_minmax_tensor(c, x, n, MM_FP8, TKV_HIP_RECIPE_PRIMARY, p));
     return launch_fp8_encode(c, x, n, p, q, out_i32);
 }
@@ -1033,6 +1066,10 @@ int launch_quant_fp8_dynamic(Ctx* c, const float* x, int64_t n, tkv_hip_qparams_
 // reference-products GEMM) instead of the codes.
 int launch_quant_fp8_dynamic_f16(Ctx* c, const float* x, int64_t n, tkv_hip_qparams_dev* p,
                                  void* h16) {
+    if (tuned(c, TKV_HIP_TUNE_QUANT_TWO_PASS) != 1) {
+        const int rc = launch_quant_resident(c, x, n, TKV_HIP_RECIPE_PRIMARY, p, h16, RES_F16);
+        if (rc != TKV_HIP_UNSUPPORTED) return rc;
+    }
     TKV_RC_TRY(launch_minmax_tensor(c, x, n, MM_FP8, TKV_HIP_RECIPE_PRIMARY, p));
     return launch_fp8_encode_as(c, x, n, p, h16, FP8_F16);
 }
