@@ -951,7 +951,7 @@ int launch_calibrate_kl(Ctx* c, const float* x, int64_t n, int64_t num_bins, int
     const size_t lds = (size_t)(((num_bins + 63) & ~63) + (target_bins > 8 ? target_bins : 8)) * 8;
     hipLaunchKernelGGL(k_kl_candidate, dim3((unsigned)(ncand > 0 ? ncand : 1)),
                        dim3(kKlCandBlock), ncand > 0 ? lds : 0, c->stream, (int)num_bins,
-                       (int)target_bins, ncand, c->cal_hist, kl, st, c->cal_arrivals + 1, out);
+                       (int)target_bins, ncand, c->cal_hist, kl, st, c->cal_arrivals + kArriveWords, out);
     TKV_LAUNCH_CHECK();
     return TKV_HIP_OK;
 }
@@ -983,7 +983,7 @@ int launch_calibrate_percentile(Ctx* c, const float* x, int64_t n, float percent
 #define TKV_RADIX(PASS)                                                                          \
     hipLaunchKernelGGL(k_radix_pass<PASS>, dim3((unsigned)grid), dim3(kHistBlock), 0, c->stream, \
                        x, n, vec, rank, symmetric ? 1 : 0, (int)nparts, c->partials, st,        \
-                       c->cal_hist, stage, staged, c->cal_arrivals + 2, out);                   \
+                       c->cal_hist, stage, staged, c->cal_arrivals + 2 * kArriveWords, out);                   \
     TKV_LAUNCH_CHECK()
     TKV_RADIX(0);
     TKV_RADIX(1);
@@ -1036,7 +1036,7 @@ static int calibrate_mse_hist(Ctx* c, const float* x, int64_t n, int nc,
                        c->stream, grid, cap, 1.0 / fixed, rows_s1, rows_n, bins);
     TKV_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_mse_bin_eval, dim3((unsigned)nc), dim3(kCalBlock), 0, c->stream, n, nc,
-                       grid, s2, bins, starts, nbins, mse, st, c->cal_arrivals + 3, out);
+                       grid, s2, bins, starts, nbins, mse, st, c->cal_arrivals + 3 * kArriveWords, out);
     TKV_LAUNCH_CHECK();
     return TKV_HIP_OK;
 }
@@ -1081,7 +1081,7 @@ int launch_calibrate_mse(Ctx* c, const float* x, int64_t n, int64_t num_candidat
         TKV_LAUNCH_CHECK();
     }
     hipLaunchKernelGGL(k_mse_reduce, dim3((unsigned)nc), dim3(kCalBlock), 0, c->stream, n, nc,
-                       grid, partial, mse, table, st, c->cal_arrivals + 3, out);
+                       grid, partial, mse, table, st, c->cal_arrivals + 3 * kArriveWords, out);
     TKV_LAUNCH_CHECK();
     return TKV_HIP_OK;
 }

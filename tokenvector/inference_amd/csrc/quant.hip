@@ -189,7 +189,7 @@ int launch_minmax_tensor(Ctx* c, const float* x, int64_t n, int mode, int recipe
         const int vec = aligned(x, 16) ? 1 : 0;
         const int64_t blocks = partial_blocks(c, vec ? n / 4 : n, vec);
         const bool nt = n * 4 > kCacheableBytes;
-        unsigned* arr = c->cal_arrivals + 0;
+        unsigned* arr = c->cal_arrivals;
 #define TKV_PARTIALS_FIN(TZ, NT)                                                           \
     hipLaunchKernelGGL((k_minmax_partials<TZ, NT, true>), dim3((unsigned)blocks),         \
                        dim3(kRedBlock), 0, c->stream, x, n, vec, c->partials, arr, mode, \

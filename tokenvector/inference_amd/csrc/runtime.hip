@@ -76,7 +76,7 @@ int ctx_create(int device, Ctx** out) {
     size_t red_bytes = sizeof(RedPartial) * kMaxReduceBlocks + 256 + sizeof(tkv_hip_qparams_dev) * 64 +
                        256 + gemv_bytes + (size_t)kGemvSplitBlocks * sizeof(unsigned) + 256 +
                        (size_t)kMaxGridSlots * 8 + (size_t)kCalHistBins * 8 +
-                       (size_t)kCalCounters * sizeof(unsigned);
+                       (size_t)kCalCounters * kArriveWords * sizeof(unsigned);
     void* red = nullptr;
     e = hipMalloc(&red, red_bytes);
     if (e != hipSuccess) {

@@ -54,6 +54,12 @@ constexpr int kMaxGridSlots = 1024;
 // Arrival counts of the calibration kernels whose last workgroup finishes
 // the call: 0 calibrate_minmax, 1 KL candidates, 2 radix passes, 3 MSE sums.
 constexpr int kCalCounters = 4;
+// An arrival count: a word for the groups and one for each group's workgroups,
+// kArriveStride words (a 256-byte line) apart.
+constexpr unsigned kArriveGroups = 16;
+constexpr unsigned kArriveStride = 64;
+constexpr unsigned kArriveFlat = 64;  // up to so many workgroups use the first word alone
+constexpr unsigned kArriveWords = (1 + kArriveGroups) * kArriveStride;
 constexpr int64_t kCalHistBins = 4096;  // the largest KL histogram
 
 struct Graph;
