@@ -12,8 +12,10 @@
 //                         three histogram passes of 11 / 11 / 10 bits, the
 //                         last block of each picking the digit; the
 //                         asymmetric form clips the min / max partials.
-//   calibrate_mse         passes over x of 16 candidate thresholds each,
-//                         summing squared quantization errors per block
+//   calibrate_mse         with many elements, one pass over x that counts
+//                         between all candidates' rounding boundaries
+//                         (k_mse_hist); else passes over x of 16 candidate
+//                         thresholds each, summing squared quantization errors per block
 //                         (f64), one block per candidate reducing those
 //                         sums, the last of them making the reference's
 //                         first-minimum pick.
