@@ -130,6 +130,37 @@ def test_value_ranges(ctx, kind):
     _check(y, a, pk, sc, b, None, m, n, k, gs)
 
 
+# One chunk of K unsplit, K splits with group sizes 128, 64 and 32.
+@pytest.mark.parametrize("m,n,k,gs", [(385, 3300, 128, 128), (200, 1030, 1024, 128),
+                                      (260, 1030, 1024, 64), (72, 2304, 2176, 32)])
+def test_scales_not_finite(ctx, m, n, k, gs):
+    """0 * scale is NaN for a NaN or infinite scale: over an activation unit
+    that is zero (rows 0 .. 63, the first 128 k), over code 8, and in sums of
+    both signs; products of one sign give an infinity."""
+    print(f"int4 planes scales {m}x{n}x{k} gs={gs}", flush=True)
+    a = O.gi_noise(m * k, 41, 1.0).reshape(m, k).copy()
+    a[:64, :128] = 0.0
+    a[66] = np.abs(a[66]) + np.float32(0.5)
+    a[67] = -a[66]
+    pk, sc = (np.array(v) for v in _weights(n, k, gs, 43))
+    pk, sc = pk.reshape(n, k // 2), sc.reshape(n, k // gs)
+    last = k // gs - 1
+    sc[0, 0] = np.nan
+    sc[3, last] = np.inf
+    sc[300, 0] = -np.inf
+    sc[n - 1, last] = np.inf
+    pk[n - 1] = 0xFF       # every code 7: infinities where the activations have one sign
+    sc[700, 0] = np.inf
+    pk[700] = 0x8F         # code 7 and code 0 in turn
+    pk[301] = 0x88         # a zero column whose scale is finite stays zero
+    a, pk, sc = (np.ascontiguousarray(v.reshape(-1)) for v in (a, pk, sc))
+    b = O.gi_noise(n, 9, 0.01)
+    y = _run(ctx, a, pk, sc, b, None, m, n, k, gs)
+    ref = _check(y, a, pk, sc, b, None, m, n, k, gs).reshape(m, n)
+    assert np.isnan(ref[0, 0]) and ref[66, n - 1] == np.inf and ref[67, n - 1] == -np.inf
+    assert np.isfinite(ref[:, 301]).all()
+
+
 def test_exact_where_the_reference_is(ctx):
     """Dyadic activations, scales and biases: every partial sum of the
     reference is exact, so every output is its bit for bit."""

@@ -23,8 +23,11 @@
 // So all sums inside a group are exact, and an output sees np roundings per
 // group (the f64 MFMA form: one per element and group).  Units that hold an
 // infinity, a NaN or an element below 2^-38 of the maximum that is not a
-// multiple of 2^(E - 56) are flagged, and the workgroups whose rows meet one
-// run their tile on the f64 MFMA instead.
+// multiple of 2^(E - 56) are flagged, and so are 64 columns x 128 k of W with a
+// scale that is not finite (0 * scale is NaN then, also where every activation
+// is zero, and the digits of one product may carry either sign).  The
+// workgroups whose rows or columns meet a flag run their tile on the f64 MFMA
+// instead.
 //
 // k_int4_planes writes A's digits and W's codes as MFMA fragments (1 KB per
 // 32 rows x 32 k, in lane order), so that the GEMM copies them to LDS with
@@ -91,17 +94,19 @@ __device__ __forceinline__ void transpose4(uint32_t a, uint32_t b, uint32_t c, u
 // nibbles unpack.  Rows past M are zeros.
 // The remaining blocks retile W: one (64 columns, 128 k) record each, the
 // packed bytes of lane (column c, half h) and k-step s at [c][16 s + 8 h ..],
-// columns past N code 8 (w = 0) with scale 0.
+// columns past N code 8 (w = 0) with scale 0, and flag the records that hold a
+// scale that is not finite (wflag: one word per record).
 __global__ __launch_bounds__(512) void k_int4_planes(
     const float* __restrict__ A, const uint8_t* __restrict__ Wp, const float* __restrict__ scales, int M, int N, int K, int gs,
     int units, int subs, uint8_t* __restrict__ planes, unsigned* __restrict__ meta,
-    uint8_t* __restrict__ wt) {
+    uint8_t* __restrict__ wt, unsigned* __restrict__ wflag) {
     const int nk = K / kUnitK, t = threadIdx.x;
     const int b = (int)blockIdx.x;
     if (b >= units * nk) {
         const int w = b - units * nk, nb = w / nk, g = w - nb * nk;
         const int half = K / 2, ng = K / gs, blk = nb % 4;
         uint8_t* rec = wt + ((int64_t)(nb / 4) * nk + g) * (4 * kWCodes + subs * 1024);
+        int odd = 0;
         if (t < 256) {
             const int lane = t & 63, h = lane >> 5;
             const int col = nb * 64 + (t >> 7) * 32 + (lane & 31);
@@ -114,9 +119,13 @@ __global__ __launch_bounds__(512) void k_int4_planes(
             reinterpret_cast<uint4*>(rec + blk * kWCodes)[t] = make_uint4(lo.x, lo.y, hi.x, hi.y);
         } else if (t < 256 + 64 * subs) {
             const int sub = (t - 256) >> 6, c = t & 63, col = nb * 64 + c;
-            reinterpret_cast<float*>(rec + 4 * kWCodes)[(sub * 4 + blk) * 64 + c] =
+            const float sc =
                 col < N ? scales[(int64_t)col * ng + (g * kUnitK + sub * (kUnitK / subs)) / gs] : 0.0f;
+            reinterpret_cast<float*>(rec + 4 * kWCodes)[(sub * 4 + blk) * 64 + c] = sc;
+            odd = (__float_as_uint(sc) & 0x7f800000u) == 0x7f800000u;
         }
+        odd = __syncthreads_or(odd);
+        if (t == 0) wflag[((int64_t)(nb / 4) * nk + g) * 4 + blk] = odd ? kFlag : 0u;
         return;
     }
     __shared__ uint32_t s_max[8], s_lo[8], s_hi[8], s_bad[8];
@@ -274,7 +283,8 @@ __device__ void f64_block(const float* __restrict__ A, const uint8_t* __restrict
 template <int SUBS, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void k_matmul_int4_planes(
     const uint8_t* __restrict__ planes, const unsigned* __restrict__ meta,
-    const uint8_t* __restrict__ wt, const float* __restrict__ A, const uint8_t* __restrict__ Wp, const float* __restrict__ scales,
+    const uint8_t* __restrict__ wt, const unsigned* __restrict__ wflag,
+    const float* __restrict__ A, const uint8_t* __restrict__ Wp, const float* __restrict__ scales,
     const float* __restrict__ bias, float* __restrict__ Y, int M, int N, int K, int gs,
     int tiles_m, int tiles_n, int chunks, double* __restrict__ part) {
     constexpr int kWRec = wrec_bytes(SUBS), kOffW = kR * kHalfSlot;
@@ -299,13 +309,18 @@ __global__ __launch_bounds__(256, 2) void k_matmul_int4_planes(
     if (wave == 0) {
         for (int base = 0; base < ng; base += 64) {
             const int g = base + lane;
-            const unsigned m = g < ng ? meta[(int64_t)unit * nk + g0 + g] : 0u;
+            unsigned m = 0u, w = 0u;
+            if (g < ng) {
+                m = meta[(int64_t)unit * nk + g0 + g];
+                const uint4 f = reinterpret_cast<const uint4*>(wflag)[(int64_t)nt * nk + g0 + g];
+                w = f.x | f.y | f.z | f.w;
+            }
             const uint64_t live = __ballot((m & 7u) != 0u);
             if (m & 7u)
                 s_chunk[nch + __popcll(live & ((1ull << lane) - 1ull))] =
                     (unsigned)g | (m & 7u) << 12 | (m >> 8) << 16;
             nch += __popcll(live);
-            bad |= (int)(m & kFlag);
+            bad |= (int)((m | w) & kFlag);
         }
         if (lane == 0) s_chunk[kMaxChunks] = (unsigned)nch;
     }
@@ -515,6 +530,7 @@ struct PlanesArgs {
     const uint8_t* planes;
     const unsigned* meta;
     const uint8_t* wt;
+    const unsigned* wflag;
     const float* a;
     const uint8_t* wp;
     const float *scales, *bias;
@@ -527,8 +543,8 @@ template <int SUBS, bool SPLIT>
 void run_planes(Ctx* c, const PlanesArgs& g) {
     hipLaunchKernelGGL((k_matmul_int4_planes<SUBS, SPLIT>),
                        dim3((unsigned)(g.tiles_m * g.tiles_n * g.splits)), dim3(256),
-                       lds_bytes(SUBS), c->stream, g.planes, g.meta, g.wt, g.a, g.wp, g.scales,
-                       g.bias, g.y, g.m, g.n, g.k, g.gs, g.tiles_m, g.tiles_n, g.chunks, g.part);
+                       lds_bytes(SUBS), c->stream, g.planes, g.meta, g.wt, g.wflag, g.a, g.wp,
+                       g.scales, g.bias, g.y, g.m, g.n, g.k, g.gs, g.tiles_m, g.tiles_n, g.chunks, g.part);
 }
 
 template <int SUBS>
@@ -576,7 +592,7 @@ int launch_matmul_int4_planes(Ctx* c, const float* a, const uint8_t* wp, const f
     const int64_t mt = units_max * kUnitRows, nt = tiles_n * kTileCols;
     const int64_t splits = planes_splits(2 * units_max * tiles_n, nk, c->num_cus, mt, nt);
     const size_t planes_need = (size_t)(units_max * nk) * (kUnitBytes + 4);
-    const size_t wt_need = (size_t)(tiles_n * nk) * wrec_bytes(subs);
+    const size_t wt_need = (size_t)(tiles_n * nk) * (wrec_bytes(subs) + 16);
     const size_t part_need = splits > 1 ? (size_t)(splits * mt * nt) * 8 : 0;
     // inside a capture nothing can grow: the f64 kernels may need no workspace
     const size_t perm_need = perm ? (size_t)(std::min(m, mt) * k) * 4 : 0;
@@ -590,12 +606,15 @@ int launch_matmul_int4_planes(Ctx* c, const float* a, const uint8_t* wp, const f
     if (splits > 1) TKV_RC_TRY(ctx_workspace(c, 12, part_need, &part));
     unsigned* meta = reinterpret_cast<unsigned*>(static_cast<uint8_t*>(planes) +
                                                  (size_t)(units_max * nk) * kUnitBytes);
+    unsigned* wflag = reinterpret_cast<unsigned*>(static_cast<uint8_t*>(wt) +
+                                                  (size_t)(tiles_n * nk) * wrec_bytes(subs));
     for (int64_t u0 = 0; u0 < units_all; u0 += panel) {
         const int64_t units = std::min(panel, units_all - u0), row0 = u0 * kUnitRows;
         PlanesArgs g;
         g.planes = static_cast<const uint8_t*>(planes);
         g.meta = meta;
         g.wt = static_cast<const uint8_t*>(wt);
+        g.wflag = wflag;
         g.a = a + row0 * k;
         g.wp = wp;
         g.scales = scales;
@@ -618,7 +637,7 @@ int launch_matmul_int4_planes(Ctx* c, const float* a, const uint8_t* wp, const f
         }
         hipLaunchKernelGGL(k_int4_planes, dim3(pgrid), dim3(512), 0, c->stream, g.a, wp, scales, g.m,
                            (int)n, (int)k, (int)gs, (int)units, subs, static_cast<uint8_t*>(planes),
-                           meta, static_cast<uint8_t*>(wt));
+                           meta, static_cast<uint8_t*>(wt), wflag);
         TKV_LAUNCH_CHECK();
         if (subs == 4)
             run_planes_subs<4>(c, g);
