@@ -188,11 +188,22 @@ __global__ __launch_bounds__(kI4Block) void k_permute_cols(const float* __restri
     }
 }
 
-// The gather form for cols <= kPermCols: a block takes ROWS whole rows through
-// LDS, so that every line of src is read once and in order (read straight from
-// memory, each element fetches a line of its own), and reads perm once for
-// them.  8192 x 3072: 133 -> 60 us.
-constexpr int kPermCols = 16384;
+// The gather form for many elements and cols <= kPermCols: a block takes ROWS
+// whole rows through LDS, so that every line of src is read once and in order
+// (read straight from memory, each element fetches a line of its own), and reads
+// perm once for them.  Four rows per block up to 1024 columns (8192 x 768 9.3 us
+// against 11.2 with one), one above: 8192 x 3072 132 us element by element, 59
+// with four rows, 40 with one.
+//   A block's row takes as long as it is wide (~1.1 us per 1024 columns), so
+// with few elements, which the caches hold, element by element is faster (3.8 us
+// up to ~2^20 elements; 1 x 3072 3.8 against 4.5, 100 x 8192 4.3 against 10.6).
+// perm_rows_from is where the two cross: 300 .. 400 rows of 3072, 250 .. 300 of
+// 4096, 200 .. 250 of 8192; of 16384, 512 rows 49 us against 38, 700 67 against
+// 72, 1024 101 against 74.
+constexpr int kPermCols = 16384, kPermFour = 1024;
+inline int64_t perm_rows_from(int64_t cols) {
+    return cols <= 4096 ? 1 << 20 : cols <= 8192 ? 7 << 18 : 12 << 20;
+}
 
 template <int ROWS>
 __global__ __launch_bounds__(kI4Block) void k_permute_rows(const float* __restrict__ src,
@@ -973,8 +984,8 @@ int launch_int4_dequantize(Ctx* c, const void* packed, bool in32, int64_t rows, 
 int launch_permute_cols(Ctx* c, const float* src, int64_t rows, int64_t cols, const int64_t* perm,
                         bool inverse, float* out) {
     if (rows * cols <= 0) return TKV_HIP_OK;
-    if (!inverse && cols <= kPermCols) {
-        const bool four = cols <= kPermCols / 4;
+    if (!inverse && cols <= kPermCols && rows * cols >= perm_rows_from(cols)) {
+        const bool four = cols <= kPermFour;
         int64_t blocks = ceil_div(rows, (int64_t)(four ? 4 : 1));
         if (blocks > (int64_t)c->num_cus * 8) blocks = (int64_t)c->num_cus * 8;
         const unsigned lds = (unsigned)(cols * 4 * (four ? 4 : 1));
