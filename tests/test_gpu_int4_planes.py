@@ -161,6 +161,40 @@ def test_scales_not_finite(ctx, m, n, k, gs):
     assert np.isfinite(ref[:, 301]).all()
 
 
+# Unsplit with group sizes 128, 64 and 32 (ragged rows and columns, a bias), K
+# splits with 128 and 32.
+@pytest.mark.parametrize("m,n,k,gs", [(385, 3300, 128, 128), (1000, 1030, 384, 64),
+                                      (1300, 1030, 384, 32), (200, 1030, 1024, 128),
+                                      (72, 2304, 2176, 32)])
+@pytest.mark.parametrize("kind", ["one", "some", "all", "special"])
+def test_flagged_chunks(ctx, m, n, k, gs, kind):
+    """Values that the planes do not hold in one chunk of K, in some, in all of
+    them: those chunks go through the f64 MFMA, the others through the planes."""
+    print(f"int4 planes flags {kind} {m}x{n}x{k} gs={gs}", flush=True)
+    a = O.gi_noise(m * k, 51, 1.0).reshape(m, k).copy()
+    small = np.float32(1.2345e-13)  # 43 orders below the maximum
+    if kind == "one":
+        a[m - 1, k - 1] = small
+    elif kind == "some":
+        a[5, 3] = small
+        a[40, k - 100] = -small
+        a[64:128, k // 2:] = 0.0
+        a[m - 3, k // 3] = np.inf
+    elif kind == "all":
+        a[::32, ::64] = small
+    else:
+        a[5, 100] = np.inf
+        a[5, k - 28] = -np.inf
+        a[65, 17] = np.nan
+        a[m - 1, k - 1] = -np.inf
+    a = np.ascontiguousarray(a.reshape(-1))
+    pk, sc = _weights(n, k, gs, 53)
+    b = O.gi_noise(n, 9, 0.01)
+    y = _run(ctx, a, pk, sc, b, None, m, n, k, gs)
+    _check(y, a, pk, sc, b, None, m, n, k, gs)
+    assert np.array_equal(y, _run(ctx, a, pk, sc, b, None, m, n, k, gs), equal_nan=True)
+
+
 def test_exact_where_the_reference_is(ctx):
     """Dyadic activations, scales and biases: every partial sum of the
     reference is exact, so every output is its bit for bit."""

@@ -26,8 +26,8 @@
 // multiple of 2^(E - 56) are flagged, and so are 64 columns x 128 k of W with a
 // scale that is not finite (0 * scale is NaN then, also where every activation
 // is zero, and the digits of one product may carry either sign).  The
-// workgroups whose rows or columns meet a flag run their tile on the f64 MFMA
-// instead.
+// workgroups whose rows or columns meet a flag run that chunk of K on the f64
+// MFMA instead.
 //
 // k_int4_planes writes A's digits and W's codes as MFMA fragments (1 KB per
 // 32 rows x 32 k, in lane order), so that the GEMM copies them to LDS with
@@ -231,49 +231,15 @@ constexpr int kHalfSlot = 8192;
 // blocks, then SUBS scales per column.
 constexpr int wrec_bytes(int subs) { return 4 * kWCodes + subs * kTileCols * 4; }
 constexpr int lds_bytes(int subs) { return kR * kHalfSlot + wrec_bytes(subs) + 4 * (kMaxChunks + 1); }
+static_assert(kTileRows * kTileCols * 8 <= kR * kHalfSlot + wrec_bytes(1), "f64 tile within the ring");
 
-// One 32 x 32 block of outputs on the f64 MFMA over k in [kbeg, kend), for
-// tiles that meet a flagged unit; the operand order of k_matmul_int4_regs
-// (lane quad q takes k0 + 8 q .. + 7 of each 32).  Rows past M and columns
-// past N read the last one.
-__device__ void f64_block(const float* __restrict__ A, const uint8_t* __restrict__ Wp,
-                          const float* __restrict__ scales, int M, int N, int K, int gs, int row0,
-                          int col0, int kbeg, int kend, int lane, f64x4 (&acc)[2][2]) {
-    const int l16 = lane & 15, q = lane >> 4, half = K / 2, ng = K / gs;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-    for (int k0 = kbeg; k0 < kend; k0 += 32) {
-        const int kk = k0 + 8 * q;
-        float a[2][8];
-        uint32_t w[2];
-        double sc[2];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const float* ar = A + (int64_t)min(row0 + 16 * i + l16, M - 1) * K;
-#pragma unroll
-            for (int e = 0; e < 8; e++) a[i][e] = ar[kk + e];
-            const int col = min(col0 + 16 * i + l16, N - 1);
-            w[i] = *reinterpret_cast<const uint32_t*>(Wp + (int64_t)col * half + kk / 2);
-            sc[i] = (double)scales[(int64_t)col * ng + kk / gs];
-        }
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            double x[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                x[i] = (double)a[i][e];
-                b[i] = (double)((int)((w[i] >> (4 * e)) & 15) - 8) * sc[i];
-            }
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i], b[j], acc[i][j], 0, 0, 0);
-        }
-    }
-}
+// What a lane loads for 32 k of the f64 form: 8 k (lane quad q takes 8 q .. + 7)
+// of 2 rows of A and of 4 columns of W with their scales.
+struct F64Raw {
+    float4 a[2][2];
+    uint32_t w[4];
+    float sc[4];
+};
 
 // y (or, SPLIT, the f64 partials of K chunks [z chunks, (z + 1) chunks)) of one
 // 32 x 256 tile per workgroup.  SUBS = 128 / gs (1 for gs >= 128) folds per
@@ -305,7 +271,8 @@ __global__ __launch_bounds__(256, 2) void k_matmul_int4_planes(
     const int unit = mt / 2;
     // the chunks of this tile that have any digits, as chunk | np << 12 |
     // (E + 512) << 16, built by wave 0; their count at the end
-    int nch = 0, bad = 0;
+    // and, from the list's end, the flagged chunks
+    int nch = 0, nbad = 0;
     if (wave == 0) {
         for (int base = 0; base < ng; base += 64) {
             const int g = base + lane;
@@ -315,17 +282,21 @@ __global__ __launch_bounds__(256, 2) void k_matmul_int4_planes(
                 const uint4 f = reinterpret_cast<const uint4*>(wflag)[(int64_t)nt * nk + g0 + g];
                 w = f.x | f.y | f.z | f.w;
             }
-            const uint64_t live = __ballot((m & 7u) != 0u);
-            if (m & 7u)
-                s_chunk[nch + __popcll(live & ((1ull << lane) - 1ull))] =
+            const bool bad = ((m | w) & kFlag) != 0u, has = !bad && (m & 7u) != 0u;
+            const uint64_t live = __ballot(has), bads = __ballot(bad), below = (1ull << lane) - 1ull;
+            if (has)
+                s_chunk[nch + __popcll(live & below)] =
                     (unsigned)g | (m & 7u) << 12 | (m >> 8) << 16;
+            if (bad) s_chunk[kMaxChunks - 1 - nbad - __popcll(bads & below)] = (unsigned)g;
             nch += __popcll(live);
-            bad |= (int)((m | w) & kFlag);
+            nbad += __popcll(bads);
         }
-        if (lane == 0) s_chunk[kMaxChunks] = (unsigned)nch;
+        if (lane == 0) s_chunk[kMaxChunks] = (unsigned)(nch | nbad << 16);
     }
-    bad = __syncthreads_or(bad);
+    __syncthreads();
     nch = __builtin_amdgcn_readfirstlane((int)s_chunk[kMaxChunks]);
+    nbad = nch >> 16;
+    nch &= 0xffff;
     const int64_t ntc = (int64_t)tiles_n * kTileCols;  // columns of the split partials
     double* __restrict__ mine = SPLIT ? part + (int64_t)z * tiles_m * kTileRows * ntc : nullptr;
     auto store = [&](int row, int col, double a, double b) {
@@ -334,26 +305,6 @@ __global__ __launch_bounds__(256, 2) void k_matmul_int4_planes(
         else if (row < M && col < N)
             __builtin_nontemporal_store((float)(a + b), Y + (int64_t)row * N + col);
     };
-    if (bad) {
-        for (int blk = wave; blk < kTileCols / 32; blk += 4) {
-            const int row0 = mt * kTileRows, col0 = nt * kTileCols + blk * 32;
-            f64x4 acc[2][2];
-            f64_block(A, Wp, scales, M, N, K, gs, row0, col0, g0 * kUnitK, g1 * kUnitK,
-                            lane, acc);
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int col = col0 + 16 * j + (lane & 15);
-                const double bb = bias && col < N ? (double)bias[col] : 0.0;
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        store(row0 + 16 * i + (lane >> 4) + 4 * e, col, acc[i][j][e], bb);
-            }
-        }
-        return;
-    }
-
     double acc[2][16];
 #pragma unroll
     for (int j = 0; j < 2; j++)
@@ -511,6 +462,86 @@ __global__ __launch_bounds__(256, 2) void k_matmul_int4_planes(
 #pragma unroll
     for (int r = 0; r < 16; r++)
         acc[1][r] = __builtin_fma((double)((hi[1][r] << 8) + lo[1][r]), wlast, acc[1][r]);
+    // The flagged chunks: the wave's 32 x 64 outputs on the f64 MFMA, each 32 k
+    // loaded while the 32 before multiply; rows past M and columns past N read the
+    // last one.  Then through LDS to the layout of acc.  Bound by the f64 matrix
+    // rate of the tile's own CU, 7 us a chunk.  No flag / one element flagged / every
+    // unit flagged, against the f64 GEMM for any values: 2048 x 2304 x 768 39.8 /
+    // 38.9 / 174 us against 140, 300 x 2304 x 768 19.5 / 29.1 / 67 against 36 (90
+    // tiles), 2048 x 768 x 3072 53 / 62 / 242 against 196, 8192 x 3072 x 768 135 /
+    // 133 / 672 against 654.  (With the tile's whole K on the f64 MFMA: one element
+    // 84, 82, 298 and 157 us.)
+    if (nbad > 0) {
+        const int l16 = lane & 15, quad = lane >> 4, ngrp = K / gs;
+        const int col0 = nt * kTileCols + wave * 64;
+        const float* arow[2];
+        const uint8_t* wcol[4];
+        const float* scol[4];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            arow[i] = A + (int64_t)min(mt * kTileRows + 16 * i + l16, M - 1) * K;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t col = min(col0 + 16 * j + l16, N - 1);
+            wcol[j] = Wp + col * (K / 2);
+            scol[j] = scales + col * ngrp;
+        }
+        auto load = [&](int step, F64Raw& r) {
+            const int g = (int)(chunk_at(kMaxChunks - 1 - step / 4) & 0xfffu);
+            const int k0 = (g0 + g) * kUnitK + 32 * (step % 4), kk = k0 + 8 * quad;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                r.a[i][0] = *reinterpret_cast<const float4*>(arow[i] + kk);
+                r.a[i][1] = *reinterpret_cast<const float4*>(arow[i] + kk + 4);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                r.w[j] = *reinterpret_cast<const uint32_t*>(wcol[j] + kk / 2);
+                r.sc[j] = scol[j][k0 / gs];
+            }
+        };
+        f64x4 fa[2][4];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) fa[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+        F64Raw next;
+        load(0, next);
+        for (int step = 0; step < 4 * nbad; step++) {
+            const F64Raw r = next;
+            if (step + 1 < 4 * nbad) load(step + 1, next);
+            const float* av[2] = {reinterpret_cast<const float*>(r.a[0]),
+                                  reinterpret_cast<const float*>(r.a[1])};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                double b[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    b[j] = (double)((int)((r.w[j] >> (4 * e)) & 15) - 8) * (double)r.sc[j];
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        fa[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av[i][e], b[j],
+                                                                       fa[i][j], 0, 0, 0);
+            }
+        }
+        __syncthreads();  // every wave is past its last read of the ring
+        double* s_f = reinterpret_cast<double*>(smem) + wave * (kTileRows * 64);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    s_f[(16 * i + quad + 4 * e) * 64 + 16 * j + l16] = fa[i][j][e];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                acc[j][r] += s_f[((r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * 64 + j * 32 + (lane & 31)];
+    }
     // D layout: lane l, register r holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
 #pragma unroll
     for (int j = 0; j < 2; j++) {
