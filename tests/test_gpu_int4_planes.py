@@ -1,7 +1,7 @@
 """GPU parity of the digit-plane INT4 GEMM (csrc/int4_planes.hip: products of
 at least 1.6e8 multiply-adds, or 2.6e8 / 3.5e8 with group sizes 64 / 32 and no
-column permutation; K % 128 == 0, group sizes 32, 64 and multiples of 128)
-against the CPU oracle.
+column permutation, more where the columns are few (csrc/int4.hip, planes_pay);
+K % 128 == 0, group sizes 32, 64 and multiples of 128) against the CPU oracle.
 
 Every sum inside a group is exact there, and each output sees at most 4
 roundings per group and 128 k, so the bound of the f64 form holds as it is:
@@ -78,17 +78,20 @@ def test_shapes(ctx, m, n, k, gs, perm, bias):
     assert np.array_equal(y, _run(ctx, a, pk, sc, b, p, m, n, k, gs))
 
 
-def test_row_panels(ctx):
-    """K = 16384: the planes of 2176 rows take two passes."""
-    m, n, k, gs = 2176, 40, 16384, 128
-    print(f"int4 planes {m}x{n}x{k}", flush=True)
+@pytest.mark.parametrize("n,perm", [(40, False), (130, False), (130, True)])
+def test_row_panels(ctx, n, perm):
+    """K = 16384: the planes of 2176 rows take two passes (40 columns are too few
+    for the planes)."""
+    m, k, gs = 2176, 16384, 128
+    print(f"int4 planes {m}x{n}x{k} perm={perm}", flush=True)
     a = O.gi_noise(m * k, 1, 1.0)
     pk, sc = _weights(n, k, gs, 2)
     b = O.gi_noise(n, 9, 0.01)
-    y = _run(ctx, a, pk, sc, b, None, m, n, k, gs).reshape(m, n)
+    p = np.random.default_rng(n).permutation(k).astype(np.int64) if perm else None
+    y = _run(ctx, a, pk, sc, b, p, m, n, k, gs).reshape(m, n)
     rows = np.r_[0:2, 2046:2050, 2174:2176]
     sub = np.ascontiguousarray(a.reshape(m, k)[rows]).reshape(-1)
-    _check(y[rows].reshape(-1), sub, pk, sc, b, None, rows.size, n, k, gs)
+    _check(y[rows].reshape(-1), sub, pk, sc, b, p, rows.size, n, k, gs)
 
 
 @pytest.mark.parametrize("kind", ["digits", "wide", "zeros", "special", "tiny"])

@@ -1019,6 +1019,34 @@ int launch_int4_split_sum(Ctx* c, const double* part, int splits, int64_t mt, in
     return TKV_HIP_OK;
 }
 
+// Prefill on the INT8 MFMA through digit planes, or the f64 MFMA.  The prepass
+// and the second launch cost ~8 us (~15 with a permutation), so the planes pay
+// from about 1.6e8 multiply-adds; with smaller groups, which fold more often, from
+// 2.6e8 (64) or 3.5e8 (32), unless a permutation sends the f64 form through its
+// slower gather.  f64 MFMA -> planes, N x K: 768 x 768 M = 256 17.6 -> 18.5 us, M
+// = 384 22.1 -> 20.4; 768 x 3072 M = 64 21.1 -> 21.0; group size 64, 1126 x 768 M
+// = 254 20.7 -> 23.2, M = 346 28.0 -> 23.4; 32, M = 346 28.2 -> 29.6, M = 462 32.6
+// -> 29.7.  2304 x 768 M = 2048 140 -> 39 us, 3072 x 768 M = 8192 656 -> 131 us,
+// 768 x 3072 M = 8192 permuted 4176 -> 215 us.
+//   The prepass and the 256-column tiles cost per element of A whatever N is, so
+// N has to exceed 70, 75 or 130 columns by enough to earn the fixed part: group
+// size 128, 64 x 768 M = 16384 32.0 -> 42.4, 16 x 3072 M = 16384 128 -> 193, 128 x
+// 768 M = 2048 17.7 -> 21.2, 256 x 768 M = 1000 17.3 -> 19.5, but 128 x 3072 M =
+// 1000 30.2 -> 28.0; 64, 128 x 768 M = 4096 27.6 -> 30.7; 32, 64 x 3072 M = 16384
+// 135 -> 293, 128 x 3072 M = 16384 254 -> 294, 192 x 3072 M = 2048 57 -> 41.
+// Permuted, where the f64 gather is slower still, only groups below 128 and few
+// columns need more (32, 64 x 3072 M = 1000 35.4 -> 41.4).  Over 685 shapes, M = 33
+// .. 16384, N = 16 .. 4096, K = 768 .. 16384, one that takes the planes is more
+// than 3% slower for it (32, 256 x 768 M = 4096 33.2 -> 36.6).
+static bool planes_pay(int64_t m, int64_t n, int64_t k, int64_t gs, bool perm) {
+    const double mk = (double)m * (double)k, macs = mk * (double)n;
+    const bool few = n <= 256;
+    if (perm) return macs >= (gs < 128 && few ? 2.7e8 : 1.6e8);
+    if (gs >= 128) return macs >= (few ? 2.4e8 : 1.6e8) && macs >= 1.0e8 + 70.0 * mk;
+    if (gs >= 64) return macs >= 2.6e8 && macs >= 1.7e8 + 75.0 * mk;
+    return macs >= 3.5e8 && macs >= 2.0e8 + 130.0 * mk;
+}
+
 int launch_matmul_int4(Ctx* c, const float* a, const uint8_t* wp, const float* scales,
                        const float* bias, const int64_t* perm, float* y, int64_t m, int64_t n,
                        int64_t k, int64_t gs) {
@@ -1119,18 +1147,7 @@ int launch_matmul_int4(Ctx* c, const float* a, const uint8_t* wp, const float* s
         TKV_GEMV(32)
 #undef TKV_GEMV
     }
-    // Prefill on the INT8 MFMA through digit planes.  The prepass and the
-    // second launch cost ~8 us (~15 with a permutation), so it pays from about
-    // 1.6e8 multiply-adds; with smaller groups, which fold more often, from
-    // 2.6e8 (64) or 3.5e8 (32), unless a permutation sends the f64 form
-    // through its slower gather.  f64 MFMA -> planes: 768 x 768 M = 256 17.6
-    // -> 18.5 us, M = 384 22.1 -> 20.4; 768 x 3072 M = 64 21.1 -> 21.0; group
-    // size 64, 1126 x 768 M = 254 20.7 -> 23.2, M = 346 28.0 -> 23.4; 32, M =
-    // 346 28.2 -> 29.6, M = 462 32.6 -> 29.7, permuted M = 254 39.7 -> 32.8.
-    // 2304 x 768 M = 2048 140 -> 39 us, 3072 x 768 M = 8192 656 -> 131 us,
-    // 768 x 3072 M = 8192 permuted 4174 -> 244 us.
-    const double macs = (double)m * (double)n * (double)k;
-    if (macs >= (perm || gs >= 128 ? 1.6e8 : gs >= 64 ? 2.6e8 : 3.5e8)) {
+    if (planes_pay(m, n, k, gs, perm != nullptr)) {
         const int rc = launch_matmul_int4_planes(c, a, wp, scales, bias, perm, y, m, n, k, gs);
         // no memory for the planes: the kernels below need far less
         if (!no_room(rc)) return rc;
