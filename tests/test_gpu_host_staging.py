@@ -1,8 +1,8 @@
-"""The INT8 GEMM's host mirror (csrc/capi.hip): int32 lists packed into, and
-results copied out of, a staging buffer of two 256 KB halves.  Sizes around a
-half and around the 16 codes that one packing step takes; codes at and past
-the int8 range at the first, middle and last place; a refused call followed by
-a good one on the same context."""
+"""The INT8 GEMM's host mirror (csrc/capi.hip): int32 lists packed into one
+buffer up to 1 MB, and above that into a staging buffer of two 256 KB halves.
+Sizes around both and around the 16 codes that one packing step takes; codes at
+and past the int8 range at the first, middle and last place; a refused call
+followed by a good one on the same context."""
 import ctypes as C
 
 import numpy as np
@@ -12,11 +12,12 @@ from tokenvector.inference_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
-# one code; K below, at and past 16; rows split over halves (K = 300 000 bytes
-# spans two); packed bytes of exactly one half (256 x 1024); results of one
-# half exactly (256 x 256 f32), one value more, and many halves
+# one code; K below, at and past 16; packed bytes of exactly 1 MB (1024 x 1024)
+# and of one row more (the first that goes through the halves); rows split over
+# halves (11 rows of K = 100 000); many halves
 SHAPES = [(1, 1, 1), (3, 5, 15), (2, 7, 17), (256, 256, 1024), (257, 256, 1023), (1, 65537, 16),
-          (300, 1000, 131), (5, 9, 100000), (1030, 2304, 768)]
+          (300, 1000, 131), (5, 9, 100000), (1030, 2304, 768), (1024, 3, 1024), (1025, 512, 1024),
+          (3, 1025, 1020), (5, 11, 100000)]
 
 
 def _accum(a, w, m, n, k):

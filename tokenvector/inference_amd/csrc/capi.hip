@@ -88,11 +88,22 @@ int pack_codes(const int32_t* src, int64_t rows, int64_t k, int64_t ldk, int8_t 
     return pack_span(src, k, ldk, bias, 0, rows * ldk, out.data());
 }
 
-// upload() of packed codes, packed half by half into the context's staging
-// buffer, so that packing a part runs while the part before it is copied.
+// upload() of packed codes.  More than 1 MB is packed half by half into the staging
+// buffer, so that packing a part runs while the part before it is copied; less is
+// packed into `keep` and copied as it is, without the events and the pinned
+// copies' own start.  Graph node, us, all through the halves -> this rule: 1 x 1 x
+// 1 72 -> 40, 1 x 64 x 1024 80 -> 60, 256 x 256 x 256 112 -> 71, 1 x 512 x 1024
+// 121 -> 102; 1 MB (1 x 1024 x 1024) 163 against 163, 4 MB 420 against 475, 1024 x
+// 768 x 3072 792 against 1084.
+constexpr int64_t kStageFrom = 4 * (int64_t)Ctx::kStageHalf;
+
 int upload_codes(Ctx* c, int slot, const int32_t* src, int64_t rows, int64_t k, int64_t ldk,
-                 void** d) {
+                 std::vector<int8_t>& keep, void** d) {
     const int64_t bytes = rows * ldk;
+    if (bytes <= kStageFrom) {
+        TKV_RC_TRY(pack_codes(src, rows, k, ldk, 0, keep));
+        return upload(c, slot, keep.data(), keep.size(), d);
+    }
     TKV_RC_TRY(ctx_workspace(c, slot, (size_t)bytes, d));
     for (int64_t off = 0; off < bytes; off += (int64_t)Ctx::kStageHalf) {
         const int64_t len = std::min<int64_t>(bytes - off, (int64_t)Ctx::kStageHalf);
@@ -103,35 +114,6 @@ int upload_codes(Ctx* c, int slot, const int32_t* src, int64_t rows, int64_t k, 
                                    hipMemcpyHostToDevice, c->stream));
         TKV_RC_TRY(ctx_stage_sent(c));
     }
-    return TKV_HIP_OK;
-}
-
-// download() through the staging buffer: a part is copied out of one half
-// while the next part arrives in the other.
-int download_staged(Ctx* c, void* h, const void* d, size_t bytes) {
-    size_t done = 0, asked = 0;
-    int in_flight = 0;
-    char* half[2];
-    size_t len[2];
-    while (done < bytes) {
-        while (asked < bytes && in_flight < 2) {
-            const int i = c->stage_at;
-            TKV_RC_TRY(ctx_stage_next(c, reinterpret_cast<void**>(&half[i])));
-            len[i] = std::min(bytes - asked, Ctx::kStageHalf);
-            TKV_HIP_TRY(hipMemcpyAsync(half[i], static_cast<const char*>(d) + asked, len[i],
-                                       hipMemcpyDeviceToHost, c->stream));
-            TKV_RC_TRY(ctx_stage_sent(c));
-            asked += len[i];
-            in_flight++;
-        }
-        const int i = in_flight == 2 ? c->stage_at : c->stage_at ^ 1;  // the older one
-        TKV_HIP_TRY(hipEventSynchronize(c->stage_event[i]));
-        memcpy(static_cast<char*>(h) + done, half[i], len[i]);
-        done += len[i];
-        in_flight--;
-    }
-    TKV_HIP_TRY(hipStreamSynchronize(c->stream));
-    c->stage_used[0] = c->stage_used[1] = false;
     return TKV_HIP_OK;
 }
 
@@ -161,10 +143,12 @@ int host_gemm_i8(const int32_t* pa, const int32_t* pw, const float* pbias, int64
     int64_t ldk = (k + ka - 1) / ka * ka;  // zero-padded: no repack in the launcher
     void *da, *dw, *dsmall, *dy;
     // Host work bounds this call: packing at the rate that int32 codes are
-    // read, the copies beside it (graph node 256 x 2304 x 768: 888 -> 459 us
-    // against packing code by code into vectors and pageable copies).
-    TKV_RC_TRY(upload_codes(c, WS_A, pa, m, k, ldk, &da));
-    TKV_RC_TRY(upload_codes(c, WS_W, pw, n, k, ldk, &dw));
+    // read, the copies beside it (graph node 256 x 2304 x 768: 883 -> 425 us
+    // against packing code by code).  The result goes straight to the caller's
+    // pages: through the halves, 4096 x 4096 x 128 took 5.3 ms against 4.2.
+    std::vector<int8_t> ha, hw;
+    TKV_RC_TRY(upload_codes(c, WS_A, pa, m, k, ldk, ha, &da));
+    TKV_RC_TRY(upload_codes(c, WS_W, pw, n, k, ldk, hw, &dw));
     // small arrays: [scale_a][scales_w (n)][bias (n)]
     std::vector<float> small(1 + 2 * (size_t)n, 0.0f);
     small[0] = scale_a;
@@ -186,7 +170,9 @@ int host_gemm_i8(const int32_t* pa, const int32_t* pw, const float* pbias, int64
     ep.k_logical = k;  // rows are zero padded to ldk
     TKV_RC_TRY(launch_gemm_i8(c, static_cast<int8_t*>(da), static_cast<int8_t*>(dw), m, n, ldk,
                               ep, dy));
-    return download_staged(c, py, dy, ybytes);
+    TKV_RC_TRY(download(c, py, dy, ybytes));
+    c->stage_used[0] = c->stage_used[1] = false;  // the stream has been waited for
+    return TKV_HIP_OK;
 }
 
 // mult = sa * sw / sy of the QLinearMatMul node (session.tkv:2024-2027).

@@ -102,8 +102,9 @@ struct Ctx {
     static constexpr int kSlots = 16;
     void* ws[kSlots] = {};
     size_t ws_bytes[kSlots] = {};
-    // Staging of the INT8 GEMM's host mirror: two halves of host memory, used
-    // in turn, each with the event of the last copy that reads or fills it.
+    // Staging of the INT8 GEMM's host mirror (codes on their way to the device):
+    // two halves of host memory, used in turn, each with the event of the last
+    // copy that reads it.
     static constexpr size_t kStageHalf = 256 << 10;
     char* stage = nullptr;
     bool stage_pinned = false;  // pageable where no pinned memory could be had
@@ -138,7 +139,7 @@ int ctx_get(int64_t handle, Ctx** out);
 // Refuses to grow while the context's stream is being captured.
 int ctx_workspace(Ctx* c, int slot, size_t bytes, void** out);
 // The next half of the staging buffer, after the last copy that used it;
-// ctx_stage_sent marks the copy just queued from or to it.
+// ctx_stage_sent marks the copy just queued from it.
 int ctx_stage_next(Ctx* c, void** half);
 int ctx_stage_sent(Ctx* c);
 // Byte fill of [dst, dst + bytes) on the context's stream (a kernel).
