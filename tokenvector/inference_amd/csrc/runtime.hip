@@ -223,9 +223,14 @@ int ctx_stage_next(Ctx* c, void** half) {
 }
 
 int ctx_stage_sent(Ctx* c) {
-    // used from here on, also if the record fails: the next wait then reports it
+    const hipError_t e = hipEventRecord(c->stage_event[c->stage_at], c->stream);
+    if (e != hipSuccess) {
+        // a wait on an event that holds no record, or an earlier one, returns at
+        // once: the copy is waited for here instead
+        (void)hipStreamSynchronize(c->stream);
+        return fail_hip(e, "hipEventRecord(staging)", __FILE__, __LINE__);
+    }
     c->stage_used[c->stage_at] = true;
-    TKV_HIP_TRY(hipEventRecord(c->stage_event[c->stage_at], c->stream));
     c->stage_at ^= 1;
     return TKV_HIP_OK;
 }
