@@ -14,9 +14,12 @@ pytestmark = pytest.mark.gpu
 
 # one tile, ragged tiles, 256 tiles of 64x64 exactly, K of one and three slices
 # (64x64); K % 256 == 128 and more tiles than CUs (64x128); one and two rounds
-# (128x128); K % 256 == 128 past them (64x128 of 4 waves, warp-specialised)
+# (128x128 from three slices on); K % 256 == 128 past them (64x128 of 4
+# waves, warp-specialised); one round more with 128x128 tiles than with 128x192
+# (warp-specialised)
 SHAPES = [(33, 1, 256), (65, 129, 768), (1024, 1024, 256), (700, 1500, 384), (1100, 1900, 256),
-          (3001, 769, 256), (3001, 2304, 512), (3001, 769, 384), (2050, 2304, 128)]
+          (1100, 1900, 768), (3001, 769, 256), (3001, 2304, 512), (3001, 2304, 768),
+          (3001, 769, 384), (2050, 2304, 128), (4100, 2300, 768)]
 
 
 @pytest.fixture(scope="module")

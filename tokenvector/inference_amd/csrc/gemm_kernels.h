@@ -1041,19 +1041,27 @@ static inline int pick_cfg(Ctx* c, int64_t m, int64_t n, int64_t ldk, bool f8) {
     //            2304x768 M = 300 9.8 -> 8.6
     //   64x128   768x3072 M = 2048 22.7 -> 21.2 (FP8 ref. 44.4 -> 40.9, qlinear
     //            18.6 -> 15.4)
-    // then 128x128 or the warp-specialised 128x192 by rounds over the CUs, a
-    // round of the smaller tile taking 0.77 of the larger's (measured 0.68 ..
-    // 0.79): 768x3072 M = 3001 (144 tiles against 96) qlinear 24.1 -> 21.3,
-    // 2304x768 M = 3001 (432 in two rounds against 288 in two) 22.8 -> 19.4;
-    // 128x192 stays for 2304x768 M = 2048 (14.9 against 18.9), 3072x768 M =
-    // 3001 (23.9 against 26.6) and large M.
+    // then 128x128 in place of the warp-specialised 128x192 where it takes as many
+    // rounds over the CUs: 768x3072 M = 3001 (144 tiles against 96) qlinear 24.1 ->
+    // 21.3, 2304x768 M = 3001 (432 in two rounds against 288 in two) 22.8 -> 19.4.
+    // 128x192 stays for 2304x768 M = 2048 (14.9 against 18.9), 3072x768 M = 3001
+    // (23.9 against 26.6) and all of one more round: 4096x1024 M = 6000 (6 against
+    // 5) int8 56 against 62, FP8 ref. 87 against 109.  With more than one round
+    // both are bound by the operand path, the smaller tile sooner: rows of 8 KB
+    // (FP8 ref., 4096x4096 M = 2048) 105 against 112, of 6 KB and less it is still
+    // the faster one (1536x3072 M = 2500 50.7 -> 48.6).  One or two slices leave no
+    // chain to shorten (2000x256 M = 1800 qlinear 6.9 against 7.2, 4096x256 M = 1024
+    // FP8 ref. 14.5 against 15.1).
     const int64_t ncu = c->num_cus;
     const bool wide_k = ldk % 256 == 0;
     if (wide_k && tiles_of<Cfg12>(m, n) <= ncu) return 12;
     if (tiles_of<Cfg14>(m, n) <= ncu) return 14;
     const int64_t t2 = tiles_of<Cfg2>(m, n);
     // (the FP8 policy holds a whole slice's fragments: 4-12% slower on it)
-    if (wide_k && !f8 && 77 * ceil_div(tiles_of<Cfg13>(m, n), ncu) < 100 * ceil_div(t2, ncu)) return 13;
+    const int64_t rounds = ceil_div(t2, ncu);
+    if (wide_k && !f8 && ldk > 512 && ceil_div(tiles_of<Cfg13>(m, n), ncu) == rounds &&
+        (rounds == 1 || ldk <= 6144))
+        return 13;
     // 128x192 tiles on three quarters of the CUs and up: at M = 2048, qkv's
     // 192 ran 10.2 us with cfg 2 against 11.4 (FP8) / 12.5 (INT8) with cfg 0
     return t2 * 4 >= ncu * 3 ? 2 : 0;
