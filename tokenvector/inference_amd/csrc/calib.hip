@@ -32,6 +32,7 @@
 #include <float.h>
 #include <limits.h>
 
+#include <algorithm>
 #include <utility>
 
 #include "tkv_device.h"
@@ -656,13 +657,20 @@ constexpr MsePartialsFn mse_partials_for(int ch, std::integer_sequence<int, CH..
 //   sum (y - 2 c q)^2 = sum d^2 + t (n_b t + 2 sum d),   t = s_b - 2 c q,
 // q = min((s_b + c) / (2 c), 127) (integers), where sum d^2 needs no bins: it is
 // the same for every candidate.  So one pass counts n_b and adds d per bin
-// (LDS), and nc x bins terms replace nc x n.  d is added in fixed point (2^-F,
-// F chosen so that a block's sum stays below 2^63: 2^-41 at 6.3 M elements,
-// 2^-38 at 50 M), which makes the result independent of the order; elements
+// (LDS), and nc x bins terms replace nc x n.  d is added in fixed point, which
+// makes the result independent of the order: in steps of 2^-F of the bin's width
+// (rounded up to a power of two), F from 46 up to 50 so that the sum of the
+// elements between two flushes to the block's f64 row stays below 2^63.  Elements
 // within rounding of a boundary are equally far from both codes.
+//   Error of the candidates' differences against the exact ones, 2^20 Gaussian,
+// bf16, int8- and int4-valued elements with and without outliers, relative: at
+// most 2e-15 (int4 values below an outlier: 2e-14), as the f64 sums of the passes
+// above (4e-15; 4e-14).  One step for all bins (2^-41 at 6.3 M elements, 2^-33 at
+// 2^30) gave up to 6e-14, and 4e-12 at 2^-35: values that repeat repeat their
+// rounding.
 //   f64 VALU work falls from 350 operations per element to 8 (nc = 50), which
-// leaves the two LDS atomics: 6.3 M elements, whole call, 105 -> 36 us; 50 M,
-// 579 -> 97 us.
+// leaves the two LDS atomics: 6.3 M elements, whole call, 103 -> 37 us; 50 M,
+// 575 -> 102 us (with one fixed-point step for all bins 35 and 97).
 constexpr int kMseHistMin = 16, kMseHistMax = 64;
 constexpr int kMseHistBlock = 1024;
 // At least the bins of nc candidates (the different integers c (2q + 1), and
@@ -670,15 +678,21 @@ constexpr int kMseHistBlock = 1024;
 constexpr int mse_bin_cap(int nc) { return 80 * nc + 320; }
 constexpr int mse_cells(int nc) { return 254 * nc; }
 
-// Dynamic LDS: s1 u64 [cap], counts u32 [cap], lut u32 [cells].  Block b writes
+// The log2 of a bin's width, rounded up (0 .. 8: the widest is 2 nc cells).
+__device__ __forceinline__ int mse_width_log2(int width) { return 32 - __clz(width - 1); }
+
+// Dynamic LDS: s1 i64 [cap], counts u32 [cap], lut u32 [cells].  Block b writes
 // its bins to rows b and its sum of d^2 to s2[b].  Every block reduces the min /
-// max partials and builds lut (cell j = int(y) -> bin | (j - start) << 16) for
-// itself from the marked boundaries, ~2 us; as a launch of its own, 13 us.  Block
-// 0 records starts[bin], *nbins and st.
+// max partials and builds lut (cell j = int(y) -> bin | start << 13 | log2 of the
+// width << 27) for itself from the marked boundaries, ~2 us; as a launch of its
+// own, 13 us.  Block 0 records starts[bin], *nbins and st.  The sums are
+// flushed (added to the block's row, cleared) every kMseFlush float4 per thread,
+// so that calls of up to 29 M elements on 256 CUs flush once, at the end.
+constexpr int kMseFlush = 28;
 __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
-    const float* __restrict__ x, int64_t n, int vec, int nc, int cap, double fixed, int nparts,
+    const float* __restrict__ x, int64_t n, int vec, int nc, int cap, int fixed, int nparts,
     const RedPartial* __restrict__ partials, CalibState* __restrict__ st,
-    unsigned long long* __restrict__ rows_s1, uint32_t* __restrict__ rows_n,
+    double* __restrict__ rows_s1, uint32_t* __restrict__ rows_n,
     double* __restrict__ s2, uint32_t* __restrict__ starts, int* __restrict__ nbins) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_mse[];
     unsigned long long* s_s1 = reinterpret_cast<unsigned long long*>(s_mse);
@@ -687,7 +701,8 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
     constexpr int kWords = 512, kWaves = kMseHistBlock / 64;
     static_assert(mse_cells(kMseHistMax) < 32 * kWords && kWords <= kMseHistBlock, "marks");
     __shared__ uint32_t s_mark[kWords];
-    __shared__ int s_bin[kWords], s_last[kWords], s_wbin[kWaves], s_wlast[kWaves];
+    __shared__ int s_bin[kWords], s_last[kWords], s_next[kWords];
+    __shared__ int s_wbin[kWaves], s_wlast[kWaves], s_wfirst[kWaves];
     __shared__ double s_red[kWaves];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, cells = mse_cells(nc);
     if (t < kWords) s_mark[t] = 0;
@@ -703,38 +718,50 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         atomicOr(&s_mark[e >> 5], 1u << (e & 31));
     }
     __syncthreads();
-    // per word: the boundaries up to its end, and the last of them
+    // per word: the boundaries up to its end, the last of them, and the first one
+    // past its end
     const uint32_t mark = t < kWords ? s_mark[t] : 0u;
     int cnt = __popc(mark), last = mark ? 32 * t + 31 - __clz((int)mark) : 0;
+    int first = mark ? 32 * t + __ffs((int)mark) - 1 : cells;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         const int a = __shfl_up(cnt, o, 64), b = __shfl_up(last, o, 64);
+        const int f = __shfl_down(first, o, 64);
         if (lane >= o) {
             cnt += a;
             last = last > b ? last : b;
         }
+        if (lane + o < 64) first = first < f ? first : f;
     }
     if (lane == 63) {
         s_wbin[wave] = cnt;
         s_wlast[wave] = last;
     }
+    if (lane == 0) s_wfirst[wave] = first;
+    int next = __shfl_down(first, 1, 64);
+    if (lane == 63) next = cells;
     __syncthreads();
     for (int w = 0; w < wave; w++) {
         cnt += s_wbin[w];
         last = last > s_wlast[w] ? last : s_wlast[w];
     }
+    for (int w = wave + 1; w < kWaves; w++) next = next < s_wfirst[w] ? next : s_wfirst[w];
     if (t < kWords) {
         s_bin[t] = cnt;
         s_last[t] = last;
+        s_next[t] = next;
     }
     __syncthreads();
     for (int j = t; j < cells; j += kMseHistBlock) {
         const int w = j >> 5;
-        const uint32_t m = s_mark[w], below = m & (0xffffffffu >> (31 - (j & 31)));
+        const uint32_t m = s_mark[w], upto = 0xffffffffu >> (31 - (j & 31));
+        const uint32_t below = m & upto, above = m & ~upto;
         const int bin = s_bin[w] - __popc(m) + __popc(below);
         const int start =
             below ? 32 * w + 31 - __clz((int)below) : (w > 0 ? s_last[w - 1] : 0);
-        s_lut[j] = (uint32_t)bin | (uint32_t)(j - start) << 16;
+        const int end = above ? 32 * w + __ffs((int)above) - 1 : s_next[w];
+        s_lut[j] = (uint32_t)bin | (uint32_t)start << 13 |
+                   (uint32_t)mse_width_log2(end - start) << 27;
         if (blockIdx.x == 0 && j == start) starts[bin] = (uint32_t)j;
     }
     if (blockIdx.x == 0 && t == 0) {
@@ -747,43 +774,67 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
     const double inv = (double)cells / am;
     __syncthreads();
     double acc = 0.0;
+    const uint32_t unit = (uint32_t)(1023 + fixed) << 20;  // the high word of 2^fixed
     auto add = [&](float v) {
-        const double y = (double)fabsf(v) * inv;
+        const double a = (double)fabsf(v);
         int j;
-        asm("v_cvt_i32_f64 %0, %1" : "=v"(j) : "v"(y));  // saturates; NaN -> 0
+        asm("v_cvt_i32_f64 %0, %1" : "=v"(j) : "v"(a * inv));  // saturates; NaN -> 0
         j = j < cells ? j : cells - 1;
         const uint32_t e = s_lut[j];
-        const double d = (y - (double)j) + (double)(e >> 16);
+        // one rounding, of d: y itself would be rounded to 2^-40 near its end
+        const double d = __builtin_fma(a, inv, -(double)((e >> 13) & 0x3fffu));
         acc = __builtin_fma(d, d, acc);  // NaN stays
-        const double f = __builtin_fma(d, fixed, 0x1p52);
-        atomicAdd(&s_s1[e & 0xffffu],
-                  (unsigned long long)(__double_as_longlong(f) & 0xfffffffffffffll));
-        atomicAdd(&s_n[e & 0xffffu], 1u);
+        const double f = __builtin_fma(
+            d, __hiloint2double((int)(unit - ((e >> 27) << 20)), 0), 0x1.8p52);
+        atomicAdd(&s_s1[e & 8191u],
+                  (unsigned long long)(uint32_t)__double2loint(f) |
+                      (unsigned long long)((uint32_t)__double2hiint(f) - 0x43380000u) << 32);
+        atomicAdd(&s_n[e & 8191u], 1u);
+    };
+    bool flushed = false;
+    auto flush = [&]() {
+        __syncthreads();
+        for (int k = t; k < cap; k += kMseHistBlock) {
+            double* row = rows_s1 + (int64_t)blockIdx.x * cap + k;
+            const double v = (double)(long long)s_s1[k];
+            *row = flushed ? *row + v : v;
+            s_s1[k] = 0;
+        }
+        flushed = true;
+        __syncthreads();
     };
     const int64_t stride = (int64_t)gridDim.x * kMseHistBlock;
     const int64_t tid = (int64_t)blockIdx.x * kMseHistBlock + threadIdx.x;
     const int64_t n4 = vec ? n / 4 : 0;
     const float4* __restrict__ x4 = reinterpret_cast<const float4*>(x);
-    int64_t i = tid;
-    for (; i + stride < n4; i += 2 * stride) {
-        const float4 u = x4[i], w = x4[i + stride];
-        add(u.x);
-        add(u.y);
-        add(u.z);
-        add(u.w);
-        add(w.x);
-        add(w.y);
-        add(w.z);
-        add(w.w);
+    for (int64_t part = 0; part < n4; part += kMseFlush * stride) {
+        if (part > 0) flush();
+        const int64_t end = part + kMseFlush * stride < n4 ? part + kMseFlush * stride : n4;
+        int64_t i = part + tid;
+        for (; i + stride < end; i += 2 * stride) {
+            const float4 u = x4[i], w = x4[i + stride];
+            add(u.x);
+            add(u.y);
+            add(u.z);
+            add(u.w);
+            add(w.x);
+            add(w.y);
+            add(w.z);
+            add(w.w);
+        }
+        for (; i < end; i += stride) {
+            const float4 u = x4[i];
+            add(u.x);
+            add(u.y);
+            add(u.z);
+            add(u.w);
+        }
     }
-    for (; i < n4; i += stride) {
-        const float4 u = x4[i];
-        add(u.x);
-        add(u.y);
-        add(u.z);
-        add(u.w);
+    for (int64_t part = 4 * n4; part < n; part += 4 * kMseFlush * stride) {
+        if (part > 4 * n4) flush();
+        const int64_t end = part + 4 * kMseFlush * stride < n ? part + 4 * kMseFlush * stride : n;
+        for (int64_t k = part + tid; k < end; k += stride) add(x[k]);
     }
-    for (int64_t k = 4 * n4 + tid; k < n; k += stride) add(x[k]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) acc = acc + __shfl_xor(acc, o, 64);
     if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
@@ -793,36 +844,38 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         for (int w = 0; w < kMseHistBlock / 64; w++) t = t + s_red[w];
         s2[blockIdx.x] = t;
     }
-    for (int k = threadIdx.x; k < cap; k += kMseHistBlock) {
-        rows_s1[(int64_t)blockIdx.x * cap + k] = s_s1[k];
+    flush();
+    for (int k = threadIdx.x; k < cap; k += kMseHistBlock)
         rows_n[(int64_t)blockIdx.x * cap + k] = s_n[k];
-    }
 }
 
 // bins[2 b] = n_b, bins[2 b + 1] = sum d of bin b: a block takes 32 bins, its 8
 // thread groups every eighth row.
 __global__ __launch_bounds__(kCalBlock) void k_mse_bin_sums(
-    int rows, int cap, double unfixed, const unsigned long long* __restrict__ rows_s1,
-    const uint32_t* __restrict__ rows_n, double* __restrict__ bins) {
+    int rows, int cap, int cells, int fixed, const double* __restrict__ rows_s1,
+    const uint32_t* __restrict__ rows_n, const uint32_t* __restrict__ starts,
+    const int* __restrict__ nbins, double* __restrict__ bins) {
     __shared__ double s_a[kCalBlock], s_b[kCalBlock];
-    const int b = blockIdx.x * 32 + (threadIdx.x & 31);
+    const int b = blockIdx.x * 32 + (threadIdx.x & 31), nb = *nbins;
+    const int end = b + 1 < cap ? (int)starts[b + 1] : 0;  // of bin nb - 1: cells
     double cn = 0.0, cs = 0.0;
     if (b < cap)
 #pragma unroll 4
         for (int r = threadIdx.x >> 5; r < rows; r += kCalBlock / 32) {
             cn = cn + (double)rows_n[(int64_t)r * cap + b];
-            cs = cs + (double)rows_s1[(int64_t)r * cap + b];
+            cs = cs + rows_s1[(int64_t)r * cap + b];
         }
     s_a[threadIdx.x] = cn;
     s_b[threadIdx.x] = cs;
     __syncthreads();
-    if (threadIdx.x < 32 && b < cap) {
+    if (threadIdx.x < 32 && b < nb) {
         for (int g = 1; g < kCalBlock / 32; g++) {
             cn = cn + s_a[32 * g + threadIdx.x];
             cs = cs + s_b[32 * g + threadIdx.x];
         }
         bins[2 * b] = cn;
-        bins[2 * b + 1] = cs * unfixed;
+        const int width = (b + 1 < nb ? end : cells) - (int)starts[b];
+        bins[2 * b + 1] = __builtin_ldexp(cs, mse_width_log2(width) - fixed);
     }
 }
 
@@ -995,11 +1048,10 @@ int launch_calibrate_percentile(Ctx* c, const float* x, int64_t n, float percent
 }
 
 // Below, the pass per 13 candidates is as fast: 50 candidates 2^17 elements
-// 32.9 -> 23.2 us, 32 candidates 23.3 -> 21.3; with fewer, 2^19 (16 candidates
-// 18.9 -> 22.1, 26 candidates 25.0 -> 24.7), 2^20 24.9 -> 23.9 and 33.0 -> 27.1.
-inline int64_t mse_hist_from(int nc) { return nc >= 32 ? 1 << 17 : 1 << 20; }
-// Fixed point has fewer bits for more elements; from here on f64 sums are the
-// more exact ones.
+// 32.8 -> 24.8 us, 32 candidates 23.0 -> 22.7; with fewer, 2^20 (16 candidates
+// 23.1 -> 24.4), 6.3 M 41.7 -> 30.6.
+inline int64_t mse_hist_from(int nc) { return nc >= 32 ? 1 << 17 : 1 << 21; }
+// Beyond, the passes: a block's 32-bit counts, and no use known.
 constexpr int64_t kMseHistTo = (int64_t)1 << 30;
 
 static int calibrate_mse_hist(Ctx* c, const float* x, int64_t n, int nc,
@@ -1008,20 +1060,20 @@ static int calibrate_mse_hist(Ctx* c, const float* x, int64_t n, int nc,
     int64_t blocks = ceil_div(n, (int64_t)kMseHistBlock * 4);
     if (blocks > c->num_cus) blocks = c->num_cus;
     const int grid = (int)blocks;
-    // a block's elements, each below 2^7 (the widest bin is 2 nc cells): the
-    // fixed-point sum of all of them stays below 2^63
-    const int64_t most = (ceil_div(n, 4 * blocks * kMseHistBlock) + 1) * 4 * kMseHistBlock;
-    int bits = 0;
-    while (((int64_t)1 << bits) < most) bits++;
-    const double fixed = (double)(1ull << (56 - bits < 44 ? 56 - bits : 44));
+    // the elements between two flushes, each at most 2^fixed steps: their sum stays
+    // below 2^63 (and each below the 2^51 that the f64 fma converts)
+    const int64_t most =
+        std::min(ceil_div(n, 4 * blocks * kMseHistBlock), (int64_t)kMseFlush) * 4 * kMseHistBlock + 4;
+    int fixed = 50;
+    while (most >= (int64_t)1 << (63 - fixed)) fixed--;
     const size_t need = (size_t)grid * cap * 12 + (size_t)grid * 8 + (size_t)cap * 20 +
                         (size_t)nc * 8 + 64;
     if (c->capturing && c->ws_bytes[9] < 256 + need) return TKV_HIP_UNSUPPORTED;
     CalibState* st;
     void* rest;
     TKV_RC_TRY(cal_workspace(c, need, &st, &rest));
-    auto* rows_s1 = static_cast<unsigned long long*>(rest);
-    auto* bins = reinterpret_cast<double*>(rows_s1 + (size_t)grid * cap);
+    auto* rows_s1 = static_cast<double*>(rest);
+    double* bins = rows_s1 + (size_t)grid * cap;
     double* s2 = bins + 2 * cap;
     double* mse = s2 + grid;
     auto* rows_n = reinterpret_cast<uint32_t*>(mse + nc);
@@ -1035,7 +1087,7 @@ static int calibrate_mse_hist(Ctx* c, const float* x, int64_t n, int nc,
                        rows_s1, rows_n, s2, starts, nbins);
     TKV_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_mse_bin_sums, dim3((unsigned)ceil_div(cap, 32)), dim3(kCalBlock), 0,
-                       c->stream, grid, cap, 1.0 / fixed, rows_s1, rows_n, bins);
+                       c->stream, grid, cap, cells, fixed, rows_s1, rows_n, starts, nbins, bins);
     TKV_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_mse_bin_eval, dim3((unsigned)nc), dim3(kCalBlock), 0, c->stream, n, nc,
                        grid, s2, bins, starts, nbins, mse, st, c->cal_arrivals + 3 * kArriveWords, out);
