@@ -111,9 +111,13 @@ def test_values_that_repeat(ctx):
 
 # around and past the elements between two flushes of the bins to their f64 rows
 # (28 float4 per thread of 256 x 1024), aligned and not
-@pytest.mark.parametrize("n,off", [(28 * 2 ** 20 - 4, 0), (28 * 2 ** 20, 0), (28 * 2 ** 20 + 4, 0),
-                                   (28 * 2 ** 20 + 5, 1), (57 * 2 ** 20 + 3, 0)])
-def test_flushes(ctx, n, off):
-    print(f"n={n} off={off}", flush=True)
+@pytest.mark.parametrize("n,off,clip", [(28 * 2 ** 20 - 4, 0, 0), (28 * 2 ** 20, 0, 0),
+                                        (28 * 2 ** 20 + 4, 0, 0.5), (28 * 2 ** 20 + 5, 1, 0),
+                                        (57 * 2 ** 20 + 3, 0, 0), (2 ** 21 + 7, 0, 1e-3)])
+def test_flushes(ctx, n, off, clip):
+    """Clipped: most elements in the last bin, which is added in registers."""
+    print(f"n={n} off={off} clip={clip}", flush=True)
     x = _x(n, n % 1000003)
+    if clip:
+        x = np.clip(x, -np.float32(clip), np.float32(clip))
     assert _bits(_choose(ctx, x, 20, off)) == _bits(O.calibrate_mse(x, 20))

@@ -670,7 +670,7 @@ constexpr MsePartialsFn mse_partials_for(int ch, std::integer_sequence<int, CH..
 // rounding.
 //   f64 VALU work falls from 350 operations per element to 8 (nc = 50), which
 // leaves the two LDS atomics: 6.3 M elements, whole call, 103 -> 37 us; 50 M,
-// 575 -> 102 us (with one fixed-point step for all bins 35 and 97).
+// 575 -> 108 us (with one fixed-point step for all bins 35 and 97).
 constexpr int kMseHistMin = 16, kMseHistMax = 64;
 constexpr int kMseHistBlock = 1024;
 // At least the bins of nc candidates (the different integers c (2q + 1), and
@@ -681,7 +681,7 @@ constexpr int mse_cells(int nc) { return 254 * nc; }
 // The log2 of a bin's width, rounded up (0 .. 8: the widest is 2 nc cells).
 __device__ __forceinline__ int mse_width_log2(int width) { return 32 - __clz(width - 1); }
 
-// Dynamic LDS: s1 i64 [cap], counts u32 [cap], lut u32 [cells].  Block b writes
+// Dynamic LDS: s1 i64 [cap], counts u32 [cap], lut u32 [cells + 1].  Block b writes
 // its bins to rows b and its sum of d^2 to s2[b].  Every block reduces the min /
 // max partials and builds lut (cell j = int(y) -> bin | start << 13 | log2 of the
 // width << 27) for itself from the marked boundaries, ~2 us; as a launch of its
@@ -752,7 +752,7 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         s_next[t] = next;
     }
     __syncthreads();
-    for (int j = t; j < cells; j += kMseHistBlock) {
+    for (int j = t; j <= cells; j += kMseHistBlock) {
         const int w = j >> 5;
         const uint32_t m = s_mark[w], upto = 0xffffffffu >> (31 - (j & 31));
         const uint32_t below = m & upto, above = m & ~upto;
@@ -775,24 +775,50 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
     __syncthreads();
     double acc = 0.0;
     const uint32_t unit = (uint32_t)(1023 + fixed) << 20;  // the high word of 2^fixed
+    // The two bins that whole tensors may fall into, whose adds would queue on one
+    // word: bin 0 (zeros) needs none, every candidate's t is 0 there, and the last
+    // one (clipped or constant values) is added in registers.  50 M zeros / equal
+    // values 387 / 388 -> 102 / 103 us, ReLU 227 -> 107; Gaussian 102 -> 108.
+    const uint32_t top = (uint32_t)s_bin[kWords - 1];
+    unsigned long long top_s = 0;
+    uint32_t top_n = 0;
     auto add = [&](float v) {
         const double a = (double)fabsf(v);
         int j;
         asm("v_cvt_i32_f64 %0, %1" : "=v"(j) : "v"(a * inv));  // saturates; NaN -> 0
-        j = j < cells ? j : cells - 1;
-        const uint32_t e = s_lut[j];
+        const uint32_t e = s_lut[j];  // at most cells (max|x| itself)
         // one rounding, of d: y itself would be rounded to 2^-40 near its end
         const double d = __builtin_fma(a, inv, -(double)((e >> 13) & 0x3fffu));
         acc = __builtin_fma(d, d, acc);  // NaN stays
         const double f = __builtin_fma(
             d, __hiloint2double((int)(unit - ((e >> 27) << 20)), 0), 0x1.8p52);
-        atomicAdd(&s_s1[e & 8191u],
-                  (unsigned long long)(uint32_t)__double2loint(f) |
-                      (unsigned long long)((uint32_t)__double2hiint(f) - 0x43380000u) << 32);
-        atomicAdd(&s_n[e & 8191u], 1u);
+        const unsigned long long s =
+            (unsigned long long)(uint32_t)__double2loint(f) |
+            (unsigned long long)((uint32_t)__double2hiint(f) - 0x43380000u) << 32;
+        const uint32_t b = e & 8191u;
+        if (b - 1u < top - 1u) {  // 0 < b < top
+            atomicAdd(&s_s1[b], s);
+            atomicAdd(&s_n[b], 1u);
+        } else if (b) {
+            top_s += s;
+            top_n++;
+        }
     };
     bool flushed = false;
     auto flush = [&]() {
+        if (__any(top_n != 0u)) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                top_s += __shfl_xor(top_s, o, 64);
+                top_n += __shfl_xor(top_n, o, 64);
+            }
+            if (lane == 0) {
+                atomicAdd(&s_s1[top], top_s);
+                atomicAdd(&s_n[top], top_n);
+            }
+            top_s = 0;
+            top_n = 0;
+        }
         __syncthreads();
         for (int k = t; k < cap; k += kMseHistBlock) {
             double* row = rows_s1 + (int64_t)blockIdx.x * cap + k;
@@ -1082,7 +1108,7 @@ static int calibrate_mse_hist(Ctx* c, const float* x, int64_t n, int nc,
     int64_t nparts;
     TKV_RC_TRY(launch_partials(c, x, n, 0, &nparts));
     hipLaunchKernelGGL(k_mse_hist, dim3((unsigned)grid), dim3(kMseHistBlock),
-                       (size_t)cap * 12 + (size_t)cells * 4, c->stream, x, n,
+                       (size_t)cap * 12 + (size_t)cells * 4 + 4, c->stream, x, n,
                        aligned(x, 16) ? 1 : 0, nc, cap, fixed, (int)nparts, c->partials, st,
                        rows_s1, rows_n, s2, starts, nbins);
     TKV_LAUNCH_CHECK();
