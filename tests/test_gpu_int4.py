@@ -167,10 +167,12 @@ def _gemm_bound(a, pk, sc, bias, m, n, k, gs, yref):
 # (one load step per 512 of K, at most 6 per trip: (1, 70, 3600, 8) runs two
 # trips, the second with 2 lanes of its second step inside K; (1, 33, 200, 8)
 # one part step), and (3, 50, 80, 16), whose K % 32 != 0, the per-column
-# kernel, as does every act-order form.  Larger M takes the 64 x 64 tile
-# kernel, with K split over workgroups when the tiles are few for the CUs (256
-# CUs): (70, 130, 256) in 2, (300, 768, 768) in 4, (128, 768, 3072) in 20 (the
-# last split shorter), (100, 60, 522, 18) in 4 on the LDS form (K % 8 != 0),
+# kernel, as does every act-order form.  Larger M takes the digit planes of
+# csrc/int4_planes.hip from ~1.6e8 multiply-adds on ((300, 768, 768), (128, 768,
+# 3072)) and below that the 64 x 64 tile kernel, with K split over workgroups when
+# the tiles are few for the CUs (256 CUs): (70, 130, 256) in 2, (260, 768, 768) in
+# 4, (40, 768, 3072) in 20 (the last split shorter), (100, 60, 522, 18) in 4 on the
+# LDS form (K % 8 != 0),
 # (1100, 1100, 256, 16) in 2 with more tiles than CUs; (520, 1040, 128) has too
 # few slices and no split (group scales applied per group: gs % 32 == 0), nor
 # has a group-scaled launch with 8 tiles per slice of K or more.  K % 32
@@ -181,6 +183,7 @@ GEMM_SHAPES = [(1, 100, 64, 32), (2, 64, 128, 32), (5, 37, 96, 32), (16, 200, 25
                (32, 130, 512, 128), (17, 1000, 1024, 128), (3, 50, 80, 16),
                (70, 130, 256, 64), (33, 2304, 768, 128), (300, 768, 768, 128),
                (129, 768, 3072, 32), (64, 768, 768, 128), (128, 768, 3072, 128),
+               (260, 768, 768, 128), (40, 768, 3072, 128),
                (200, 100, 512, 32), (100, 60, 522, 18), (520, 1040, 128, 32),
                (1100, 1100, 256, 16), (90, 70, 200, 8), (100, 60, 520, 8),
                (1, 70, 3600, 8), (1, 33, 200, 8)]
@@ -291,14 +294,14 @@ def test_int4_decode_gpt2_shapes(ctx, name, n, k, m):
 def test_graph_replays_int4(ctx):
     """matmul_int4_grouped on device buffers captured in one graph: M = 1
     (single-row kernel), 32 (decode kernel, K split over workgroups with
-    arrival counts), 200 (tile kernel, K split + split sum) on a 768 x 3072
-    weight and 520 (tile kernel unsplit, group scales per group) on a 256 x
-    128 one.  Replays after new activations, with eager calls of other sizes
+    arrival counts), 60 (tile kernel, K split + split sum) and 200 (digit planes,
+    K split) on a 768 x 3072 weight and 520 (tile kernel unsplit, group scales per
+    group) on a 256 x 128 one.  Replays after new activations, with eager calls of other sizes
     between them, give the eager results bit for bit; the eager results are
     within the reordering bound of the oracle."""
     say("graph replays int4")
     cases = []
-    for (n, k, gs, ms, seed) in ((768, 3072, 128, (1, 32, 200), 61), (256, 128, 32, (520,), 63)):
+    for (n, k, gs, ms, seed) in ((768, 3072, 128, (1, 32, 60, 200), 61), (256, 128, 32, (520,), 63)):
         w = _weights(n, k, seed)
         pk, sc = O.quantize_int4_grouped(w, n, k, gs)
         dw = D.DeviceBuffer.from_host(ctx, pk.astype(np.uint8))
