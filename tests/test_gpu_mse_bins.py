@@ -1,5 +1,5 @@
 """GPU parity of calibrate_mse's one-pass form (csrc/calib.hip: 16 .. 31
-candidates from 2^21 elements on, 32 .. 64 from 2^17) against the CPU oracle (engine.tkv:165-197).
+candidates from 2^21 elements on, 32 .. 39 from 2^18, 40 .. 64 from 2^17) against the CPU oracle (engine.tkv:165-197).
 
 The chosen threshold must be the oracle's: two candidates' errors differ by far
 more than the rounding of either sum except where they tie exactly, and then
@@ -50,7 +50,8 @@ def _x(n, seed, heavy=True):
 @pytest.mark.parametrize("n,nc", [(131071, 32), (131072, 31), (131072, 32), (131073, 50),
                                   (262147, 64), (262147, 65), (1048575, 31), (1048576, 16),
                                   (1048579, 31), (1048576, 15), (2100001, 17), (2100001, 64),
-                                  (2097151, 16), (2097152, 16), (2097155, 31), (2097152, 15)])
+                                  (2097151, 16), (2097152, 16), (2097155, 31), (2097152, 15),
+                                  (262143, 32), (262144, 32), (262145, 39), (131071, 40), (131072, 40)])
 def test_sizes_and_candidates(ctx, n, nc):
     """Both sides of each line of the rule; n past whole float4 groups, and x one
     float past a 16-byte boundary."""
@@ -115,7 +116,7 @@ def test_values_that_repeat(ctx):
                                         (28 * 2 ** 20 + 4, 0, 0.5), (28 * 2 ** 20 + 5, 1, 0),
                                         (57 * 2 ** 20 + 3, 0, 0), (2 ** 21 + 7, 0, 1e-3)])
 def test_flushes(ctx, n, off, clip):
-    """Clipped: most elements in the last bin, which is added in registers."""
+    """Clipped: most elements in the last bin, which has a slot per lane."""
     print(f"n={n} off={off} clip={clip}", flush=True)
     x = _x(n, n % 1000003)
     if clip:

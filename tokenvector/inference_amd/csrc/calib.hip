@@ -674,12 +674,13 @@ constexpr MsePartialsFn mse_partials_for(int ch, std::integer_sequence<int, CH..
 // rounding.
 //   f64 VALU work falls from 350 operations per element to 8 (nc = 50), which
 // leaves the two LDS atomics: 6.3 M elements, whole call, 103 -> 37 us; 50 M,
-// 575 -> 108 us (with one fixed-point step for all bins 35 and 97).
+// 575 -> 103 us (with one fixed-point step for all bins 35 and 97).
 constexpr int kMseHistMin = 16, kMseHistMax = 64;
 constexpr int kMseHistBlock = 1024;
 // At least the bins of nc candidates (the different integers c (2q + 1), and
-// one), counted for 16 .. 64: 1541 for 16, 2864 for 32, 4218 for 50, 5309 for 64.
-constexpr int mse_bin_cap(int nc) { return 80 * nc + 320; }
+// one), counted for 16 .. 64: 1541 for 16, 2864 for 32, 4218 for 50, 5309 for 64;
+// and 127 for the slots by lane of the first and the last bin.
+constexpr int mse_bin_cap(int nc) { return 80 * nc + 448; }
 constexpr int mse_cells(int nc) { return 254 * nc; }
 
 // The log2 of a bin's width, rounded up (0 .. 8: the widest is 2 nc cells).
@@ -756,6 +757,11 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         s_next[t] = next;
     }
     __syncthreads();
+    // The two bins that whole tensors may fall into, whose adds would queue on one
+    // word, have a slot per lane: the last one (clipped or constant values) top ..
+    // top + 63, bin 0 (zeros) the next 64, which nothing reads (every candidate's t
+    // is 0 there).  50 M zeros / equal values 387 / 388 -> 98 / 98 us, ReLU 227 -> 100.
+    const int top = s_bin[kWords - 1];
     for (int j = t; j <= cells; j += kMseHistBlock) {
         const int w = j >> 5;
         const uint32_t m = s_mark[w], upto = 0xffffffffu >> (31 - (j & 31));
@@ -764,7 +770,7 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         const int start =
             below ? 32 * w + 31 - __clz((int)below) : (w > 0 ? s_last[w - 1] : 0);
         const int end = above ? 32 * w + __ffs((int)above) - 1 : s_next[w];
-        s_lut[j] = (uint32_t)bin | (uint32_t)start << 13 |
+        s_lut[j] = (uint32_t)(bin ? bin : top + 64) | (uint32_t)start << 13 |
                    (uint32_t)mse_width_log2(end - start) << 27;
         if (blockIdx.x == 0 && j == start) starts[bin] = (uint32_t)j;
     }
@@ -773,19 +779,12 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         st->am = am;
         st->mn = dmn;
         st->mx = dmx;
-        *nbins = s_bin[kWords - 1] + 1;
+        *nbins = top + 1;
     }
     const double inv = (double)cells / am;
     __syncthreads();
     double acc = 0.0;
     const uint32_t unit = (uint32_t)(1023 + fixed) << 20;  // the high word of 2^fixed
-    // The two bins that whole tensors may fall into, whose adds would queue on one
-    // word: bin 0 (zeros) needs none, every candidate's t is 0 there, and the last
-    // one (clipped or constant values) is added in registers.  50 M zeros / equal
-    // values 387 / 388 -> 102 / 103 us, ReLU 227 -> 107; Gaussian 102 -> 108.
-    const uint32_t top = (uint32_t)s_bin[kWords - 1];
-    unsigned long long top_s = 0;
-    uint32_t top_n = 0;
     auto add = [&](float v) {
         const double a = (double)fabsf(v);
         int j;
@@ -796,35 +795,28 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         acc = __builtin_fma(d, d, acc);  // NaN stays
         const double f = __builtin_fma(
             d, __hiloint2double((int)(unit - ((e >> 27) << 20)), 0), 0x1.8p52);
-        const unsigned long long s =
-            (unsigned long long)(uint32_t)__double2loint(f) |
-            (unsigned long long)((uint32_t)__double2hiint(f) - 0x43380000u) << 32;
-        const uint32_t b = e & 8191u;
-        if (b - 1u < top - 1u) {  // 0 < b < top
-            atomicAdd(&s_s1[b], s);
-            atomicAdd(&s_n[b], 1u);
-        } else if (b) {
-            top_s += s;
-            top_n++;
-        }
+        const int bin = (int)(e & 8191u), slot = bin + (bin >= top ? lane : 0);
+        atomicAdd(&s_s1[slot],
+                  (unsigned long long)(uint32_t)__double2loint(f) |
+                      (unsigned long long)((uint32_t)__double2hiint(f) - 0x43380000u) << 32);
+        atomicAdd(&s_n[slot], 1u);
     };
     bool flushed = false;
     auto flush = [&]() {
-        if (__any(top_n != 0u)) {
+        __syncthreads();
+        if (wave == 0) {  // the last bin's slots into its first
+            unsigned long long s = s_s1[top + lane];
+            uint32_t c = s_n[top + lane];
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) {
-                top_s += __shfl_xor(top_s, o, 64);
-                top_n += __shfl_xor(top_n, o, 64);
+                s += __shfl_xor(s, o, 64);
+                c += __shfl_xor(c, o, 64);
             }
-            if (lane == 0) {
-                atomicAdd(&s_s1[top], top_s);
-                atomicAdd(&s_n[top], top_n);
-            }
-            top_s = 0;
-            top_n = 0;
+            s_s1[top + lane] = lane ? 0 : s;
+            s_n[top + lane] = lane ? 0 : c;
         }
         __syncthreads();
-        for (int k = t; k < cap; k += kMseHistBlock) {
+        for (int k = t; k <= top; k += kMseHistBlock) {
             double* row = rows_s1 + (int64_t)blockIdx.x * cap + k;
             const double v = (double)(long long)s_s1[k];
             *row = flushed ? *row + v : v;
@@ -875,7 +867,7 @@ __global__ __launch_bounds__(kMseHistBlock) void k_mse_hist(
         s2[blockIdx.x] = t;
     }
     flush();
-    for (int k = threadIdx.x; k < cap; k += kMseHistBlock)
+    for (int k = threadIdx.x; k <= top; k += kMseHistBlock)
         rows_n[(int64_t)blockIdx.x * cap + k] = s_n[k];
 }
 
@@ -1077,10 +1069,12 @@ int launch_calibrate_percentile(Ctx* c, const float* x, int64_t n, float percent
     return TKV_HIP_OK;
 }
 
-// Below, the pass per 13 candidates is as fast: 50 candidates 2^17 elements
-// 32.8 -> 24.8 us, 32 candidates 23.0 -> 22.7; with fewer, 2^20 (16 candidates
-// 23.1 -> 24.4), 6.3 M 41.7 -> 30.6.
-inline int64_t mse_hist_from(int nc) { return nc >= 32 ? 1 << 17 : 1 << 21; }
+// Below, the pass per 13 candidates is as fast: 2^17 elements, 50 candidates 32.6
+// -> 25.2 us, 32 candidates 22.9 -> 23.2; with fewer than 32, 2^20 (16 candidates
+// 23.1 -> 24.4), 6.3 M 41.7 -> 31.1.
+inline int64_t mse_hist_from(int nc) {
+    return nc >= 40 ? 1 << 17 : nc >= 32 ? 1 << 18 : 1 << 21;
+}
 // Beyond, the passes: a block's 32-bit counts, and no use known.
 constexpr int64_t kMseHistTo = (int64_t)1 << 30;
 
