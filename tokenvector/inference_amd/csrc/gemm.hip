@@ -94,7 +94,12 @@ int launch_gemm_qlinear(Ctx* c, const int8_t* a, const int8_t* w, int64_t m, int
     // attn_out 14.1 / 15.0 us, mlp_down (one tile of 24 slices per
     // workgroup) 29.8 / 32.4, qkv (three tiles of 6) 34.1 / 33.9, mlp_up
     // (four tiles of 6) 43.3 / 41.9.  So the GEMM sums whenever a workgroup
-    // runs one tile, or few slices in all.
+    // runs one tile, or few slices in all.  For fewer tiles than that launch_any
+    // takes the plain tile kernels, which sum in every wave; whole calls against the
+    // pre-pass there: 768x768 M = 256 5.5 / 7.6 us, M = 3001 9.2 / 10.9, 2304x768 M
+    // = 2048 12.0 / 13.2, 768x3072 M = 512 11.3 / 12.2, 4096x4096 M = 256 15.2 /
+    // 17.5; 768x3072 M = 3001 20.3 / 19.2 with zpw = 0.  (With both zero points 0
+    // the pre-pass launches nothing and would be 3-18% faster.)
     const int64_t tiles = gemm::tiles_of<gemm::Cfg2>(m, n);
     const int64_t slices = ceil_div(tiles, (int64_t)c->num_cus) * (ldk / gemm::kBK);
     if (m > gemm::kGemvMaxM && (tiles <= c->num_cus || slices <= 12)) {

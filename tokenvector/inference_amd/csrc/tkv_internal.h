@@ -266,7 +266,7 @@ int launch_matmul_int4(Ctx* c, const float* a, const uint8_t* wp, const float* s
                        const float* bias, const int64_t* perm, float* y, int64_t m, int64_t n,
                        int64_t k, int64_t gs);
 // The same on the INT8 MFMA through the activations' digit planes
-// (int4_planes.hip).  K not a multiple of 128 or above 65536, group sizes
+// (int4_planes.hip).  K not a multiple of 128 or above 16384, group sizes
 // other than 32, 64 and the multiples of 128, unaligned operands, or a capture
 // whose workspaces are too small: UNSUPPORTED, nothing launched.
 int launch_matmul_int4_planes(Ctx* c, const float* a, const uint8_t* wp, const float* scales,
