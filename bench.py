@@ -324,8 +324,8 @@ def bench_int4(ctx, D, G, ms=(1, 32, 256, 8192), gs=128):
     accumulation at decode, small-prefill (K split over workgroups) and prefill
     batches (exact products on v_mfma_f64_16x16x4_f64, peak 78.6 TFLOP/s, or from
     ~1.6e8 multiply-adds through exact digit planes on the INT8 units), the
-    symmetric weight quantizer, and GGUF Q8_0 decoding of the same weights.  Weights are quantized once, outside
-    the timed launches; 12 layers' weights are cycled so decode batches stream
+    symmetric weight quantizer, and GGUF Q8_0 decoding of the same weights.
+    Weights are quantized once, outside the timed launches; 12 layers' weights are cycled so decode batches stream
     them from HBM."""
     out = {}
     for (name, n, k) in SHAPES:

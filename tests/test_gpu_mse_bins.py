@@ -1,5 +1,6 @@
 """GPU parity of calibrate_mse's one-pass form (csrc/calib.hip: 16 .. 31
-candidates from 2^21 elements on, 32 .. 39 from 2^18, 40 .. 64 from 2^17) against the CPU oracle (engine.tkv:165-197).
+candidates from 2^21 elements on, 32 .. 39 from 2^18, 40 .. 64 from 2^17)
+against the CPU oracle (engine.tkv:165-197).
 
 The chosen threshold must be the oracle's: two candidates' errors differ by far
 more than the rounding of either sum except where they tie exactly, and then
@@ -51,7 +52,8 @@ def _x(n, seed, heavy=True):
                                   (262147, 64), (262147, 65), (1048575, 31), (1048576, 16),
                                   (1048579, 31), (1048576, 15), (2100001, 17), (2100001, 64),
                                   (2097151, 16), (2097152, 16), (2097155, 31), (2097152, 15),
-                                  (262143, 32), (262144, 32), (262145, 39), (131071, 40), (131072, 40)])
+                                  (262143, 32), (262144, 32), (262145, 39),
+                                  (131071, 40), (131072, 40)])
 def test_sizes_and_candidates(ctx, n, nc):
     """Both sides of each line of the rule; n past whole float4 groups, and x one
     float past a 16-byte boundary."""

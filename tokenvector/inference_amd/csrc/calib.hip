@@ -352,11 +352,11 @@ __global__ __launch_bounds__(kKlCandBlock) void k_kl_candidate(
 constexpr int kPctStage = 4096;
 
 // One radix pass: the digit (bits(|x|) >> shift) & (2^bits - 1) counted over
-// the elements whose higher bits equal the prefix found so far (one LDS
-// histogram per block, kKlVec float4 per lane per trip), merged into the
+// the elements whose higher bits equal the prefix found so far (LDS
+// histograms per block, kKlVec float4 per lane per trip), merged into the
 // global histogram.  The block that arrives last (arrive_last) finds the
 // digit holding the element of the wanted rank (block prefix sum over the
-// 2048 digit counts, 8 per thread), records prefix and rank in st, clears
+// 2048 digit counts, 2 per thread), records prefix and rank in st, clears
 // the histogram, and after the last pass writes the parameters.
 //   The second pass also stages the bits of every element it counts (those
 // whose top 11 bits match) in LDS and writes them to its own kPctStage-entry
@@ -397,7 +397,8 @@ __global__ __launch_bounds__(kHistBlock) void k_radix_pass(
     // if the tensor holds it so.  Four copies: 2^20 equal values 39.1 -> 28.6 us (8:
     // 28.5, but 0.1 us more for a small Gaussian).  The second also stages, with a
     // second add per element on one word whatever the values are.
-    constexpr int copies = PASS == 0 ? kRadixCopies : PASS == 1 ? 1 : 4, bins = 1 << bits, pitch = bins + 1;
+    constexpr int copies = PASS == 0 ? kRadixCopies : PASS == 1 ? 1 : 4;
+    constexpr int bins = 1 << bits, pitch = bins + 1;
     __shared__ unsigned int s_hist[copies * pitch];
     unsigned int* s_h = s_hist + ((int)threadIdx.x & (copies - 1)) * pitch;
     __shared__ uint32_t s_stage[PASS == 1 ? kPctStage : 1];
