@@ -341,7 +341,7 @@ __global__ __launch_bounds__(kKlCandBlock) void k_kl_candidate(
         else
             write_sym((double)best_bin * st->bw, out);
     }
-    arrive_clear(arrivals);
+    arrive_clear(arrivals, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -544,7 +544,7 @@ __global__ __launch_bounds__(kHistBlock) void k_radix_pass(
             }
         }
     }
-    arrive_clear(arrivals);
+    arrive_clear(arrivals, arriving);
 }
 
 // ---------------------------------------------------------------------------
@@ -941,7 +941,7 @@ __global__ __launch_bounds__(kCalBlock) void k_mse_bin_eval(
         else
             write_sym(bc >= 0 ? am * (double)(bc + 1) / (double)nc : am, out);
     }
-    arrive_clear(arrivals);
+    arrive_clear(arrivals, gridDim.x);
 }
 
 // mse[c] = (sum over the per-block partials, a fixed tree order) / n.  The
@@ -975,7 +975,7 @@ __global__ __launch_bounds__(kCalBlock) void k_mse_reduce(int64_t n, int nc, int
         else
             write_sym(bc >= 0 ? table[3 * bc] : st->am, out);
     }
-    arrive_clear(arrivals);
+    arrive_clear(arrivals, gridDim.x);
 }
 
 // Histogram passes (KL, radix): one workgroup of kHistBlock threads per CU, or as

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kRedBlock) void k_minmax_partials(const float* __re
             if (x0 != x0) dmn = dmx = (double)x0;  // nan_first
             finalize_minmax(dmn, dmx, mode, recipe, out);
         }
-        arrive_clear(arrivals);
+        arrive_clear(arrivals, gridDim.x);
     }
 }
 

@@ -134,8 +134,10 @@ __device__ __forceinline__ bool arrive_last(unsigned* counter, unsigned total) {
     return s_last != 0;
 }
 
-__device__ __forceinline__ void arrive_clear(unsigned* counter) {
-    if (threadIdx.x <= kArriveGroups)
+// Clears the words that arrive_last(counter, total) counted on: all 17 lines where
+// the first was the only one cost min / max of 256 x 768 0.04 us of 4.2.
+__device__ __forceinline__ void arrive_clear(unsigned* counter, unsigned total) {
+    if (threadIdx.x <= (total > kArriveFlat ? kArriveGroups : 0u))
         __hip_atomic_store(counter + threadIdx.x * kArriveStride, 0u, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
 }
